@@ -183,15 +183,16 @@ def one_pass(m: int, n: int, k: int) -> bool:
     return k < n - 2 and m - k <= FG_ROWS and n - k - 1 <= 256 * 512
 
 
-def gemv_bytes(m: int, n: int) -> dict:
-    """Algorithmic bytes per kernel over the column steps of one m x n
-    (m >= n) bidiagonalization, as the driver chooses them: a one-pass step
+def gemv_bytes(m: int, n: int, steps: int) -> dict:
+    """Algorithmic bytes per kernel over the first `steps` column steps of one
+    m x n (m >= n) bidiagonalization (the rest runs with the matrix in
+    registers, resident.hip), as the driver chooses them: a one-pass step
     reads its trailing block A0[k:m, k+1:n] once, 8 (m-k)(n-k-1) bytes; a
     two-pass step has a left GEMV of 8 (m-k)(n-k-1) bytes (none at a panel's
     first column after the first, whose partial sums the trailing update
     forms) and, below k = n-2, a right GEMV of 8 (m-k-1)(n-k-1)."""
     out = {"bd_fused_gemv": 0, "bd_left_gemv": 0, "bd_right_gemv": 0}
-    for k in range(n - 1):
+    for k in range(min(steps, n - 1)):
         if one_pass(m, n, k):
             out["bd_fused_gemv"] += 8 * (m - k) * (n - k - 1)
             continue
@@ -1014,7 +1015,9 @@ def main() -> int:
 
     mt, nt = max(m, n), mn
     gemv = {}
-    gb = gemv_bytes(mt, nt)
+    # steps with a GEMV launch of their own: one-pass, or a right GEMV
+    gemv_steps = int(kt["fused_gemv_launches"] + kt["right_gemv_launches"] + 0.5)
+    gb = gemv_bytes(mt, nt, gemv_steps if gemv_steps < nt - 2 else nt)
     for name, key in (("bd_fused_gemv", "fused_gemv"), ("bd_left_gemv", "left_gemv"),
                       ("bd_right_gemv", "right_gemv")):
         nbytes = gb[name]
@@ -1027,8 +1030,10 @@ def main() -> int:
                       "avg_launch_us": 1e6 * t / nl if t > 0 else None,
                       "launches_per_svd": nl, "ms_per_svd": 1e3 * t,
                       "traffic": traffic_summary(m, n, name)}
-    dom = max(gemv, key=lambda k: gemv[k]["ms_per_svd"])
-    g = gemv[dom]
+    none = {"achieved_GBs": None, "traffic": None, "algorithmic_bytes_per_launch": None,
+            "avg_launch_us": None, "launches_per_svd": 0}  # all steps in registers
+    dom = max(gemv, key=lambda k: gemv[k]["ms_per_svd"]) if gemv else None
+    g = gemv[dom] if gemv else none
     achieved = g["achieved_GBs"]
     t_bd = stage["bidiag"] / 1000.0
     out = {

@@ -34,6 +34,7 @@
 #include <cstdlib>
 
 #include "ddc_common.h"
+#include "householder.h"
 
 namespace ddc {
 
@@ -130,29 +131,6 @@ __device__ __forceinline__ double sum_strided(const double* p, int cnt, int64_t 
   }
   return acc;
 }
-
-// Householder data of the vector x with |x|^2 = sumsq and first entry x1,
-// as the reference forms it (update_scale_matcol.cl:58-82): diag =
-// -sign(x1)|x|, reflector = (x + sign(x1)|x| e1) / rl with
-// rl = sqrt(2) sqrt(|x|^2 + ||x| x1|).  A zero vector gives rl = 0 and is
-// treated as "no reflection" (the reference divides by zero there).
-struct Refl {
-  double nrm, sgn, rl;
-  __device__ __forceinline__ void make(double sumsq, double x1) {
-    nrm = sqrt(sumsq);
-    sgn = (x1 < 0) ? -1.0 : 1.0;
-    rl = sqrt(2.0) * sqrt(nrm * nrm + fabs(nrm * x1));
-  }
-  __device__ __forceinline__ double diag() const { return rl != 0.0 ? -sgn * nrm : 0.0; }
-  __device__ __forceinline__ double vec(double x, bool first) const {
-    if (rl == 0.0) return 0.0;
-    return (first ? x + sgn * nrm : x) / rl;
-  }
-  // (w^T reflector) from (w^T x) and the first entry w1 of w
-  __device__ __forceinline__ double dot(double wx, double w1) const {
-    return rl != 0.0 ? (wx + sgn * nrm * w1) / rl : 0.0;
-  }
-};
 
 // ---------------------------------------------------------------------------
 
@@ -676,70 +654,6 @@ __device__ __forceinline__ double buf_load<double>(__amdgpu_buffer_rsrc_t r, int
 template <>
 __device__ __forceinline__ double buf_load<float>(__amdgpu_buffer_rsrc_t r, int voff) {
   return (double)__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
-}
-
-// Wave sum by DPP (row-local butterflies, then the row broadcasts of gfx9),
-// in a fixed order; every lane gets lane 63's total.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_take(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, CTRL, ROWS, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), CTRL, ROWS, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-// (every lane written: no old value to set)
-template <int CTRL>
-__device__ __forceinline__ double dpp_all(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)b, CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), CTRL, 0xf, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double lane63(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)b, 63);
-  const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(b >> 32), 63);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-__device__ __forceinline__ double wave_total(double v) {
-  v += dpp_all<0xB1>(v);         // quad_perm [1,0,3,2]: pairs
-  v += dpp_all<0x4E>(v);         // quad_perm [2,3,0,1]: quads
-  v += dpp_all<0x141>(v);        // row_half_mirror: eights
-  v += dpp_all<0x140>(v);        // row_mirror: rows of 16
-  v += dpp_take<0x142, 0xA>(v);  // row_bcast:15 into rows 1, 3
-  v += dpp_take<0x143, 0xC>(v);  // row_bcast:31 into rows 2, 3: lane 63 has the total
-  return lane63(v);
-}
-// Three wave totals with their stages interleaved (independent chains).
-__device__ __forceinline__ void wave_total3(double& a, double& b, double& c) {
-  a += dpp_all<0xB1>(a);
-  b += dpp_all<0xB1>(b);
-  c += dpp_all<0xB1>(c);
-  a += dpp_all<0x4E>(a);
-  b += dpp_all<0x4E>(b);
-  c += dpp_all<0x4E>(c);
-  a += dpp_all<0x141>(a);
-  b += dpp_all<0x141>(b);
-  c += dpp_all<0x141>(c);
-  a += dpp_all<0x140>(a);
-  b += dpp_all<0x140>(b);
-  c += dpp_all<0x140>(c);
-  a += dpp_take<0x142, 0xA>(a);
-  b += dpp_take<0x142, 0xA>(b);
-  c += dpp_take<0x142, 0xA>(c);
-  a += dpp_take<0x143, 0xC>(a);
-  b += dpp_take<0x143, 0xC>(b);
-  c += dpp_take<0x143, 0xC>(c);
-  a = lane63(a);
-  b = lane63(b);
-  c = lane63(c);
-}
-
-// num / d from ir = 1/d (0 for d = 0, giving 0): q0 = num ir, then one
-// correction q0 + (num - q0 d) ir with fused multiply-adds.
-__device__ __forceinline__ double rl_quot(double num, double d, double ir) {
-  const double q0 = num * ir;
-  return fma(fma(-q0, d, num), ir, q0);
 }
 
 template <typename TS, int RPT, int D, bool PAIR>
@@ -1427,6 +1341,7 @@ static void bidiag_plan_common(ArenaPlan& p, int m, int n, int lda) {
   p.add<double>((size_t)d.nccR_max * DSTRIDE);
   p.add<double>(d.ncn_max);
   p.add<double>(d.nrn_max);
+  resident_plan(p);
 }
 
 void bidiag_plan(ArenaPlan& p, int m, int n, int lda) { bidiag_plan_common(p, m, n, lda); }
@@ -1539,6 +1454,8 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
     return fused_gemv_on() && kk < n - 2 && !(m < n && kk >= m - 1) && m - kk <= FG_ROWS &&
            n - kk - 1 <= FG_GMAX * FG_MAXCOL;
   };
+  // columns from this panel boundary on fit the register files (resident.hip)
+  int res_k = fused_gemv_on() ? resident_first<TS>(m, n, NB) : -1;
   int fusedL = 0;  // tiles of left GEMV partials the trailing update left for step k, or 0
   int nfr_prev = 0;  // groups of the previous bd_right_fin (rows of its panel dots)
   for (int k = 0; k < mn; ++k) {
@@ -1547,6 +1464,20 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
     a.t = k - a.p;
     const int nt = fusedL;
     fusedL = 0;
+    if (k == res_k) {
+      int done = 0;
+      DDC_TRY(resident_run<TS>(m, n, A, lda, alpha, beta, k, NB, ws, st, &done));
+      if (done >= mn) break;
+      // the work-groups found no room beside other work: the rest below,
+      // from panel boundary `done` (resident_run is not tried again)
+      res_k = -1;
+      k = done - 1;
+      a.ncn = (int)ceil_div(m - done, 256);
+      hipLaunchKernelGGL(bd_init<TS>, dim3(a.ncn), dim3(256), 0, st, m - done,
+                         A + done + (int64_t)done * lda, a.cvec + done, a.cnorm);
+      DDC_LAUNCHED();
+      continue;
+    }
     if (m < n && k == m - 1) {
       const int nw = (int)ceil_div(n - k - 1, FIN);
       hipLaunchKernelGGL(bd_wide_row<TS>, dim3(nw), dim3(FIN), 0, st, a);
@@ -1629,7 +1560,7 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
         // GEMV (column r0 of the updated matrix is c, from bd_right_fin)
         // when that step is a plain one: one pass over the trailing matrix
         // less per panel.
-        const bool fuse = !one_pass(r0) && r0 < n - 1 && !(m < n && r0 == m - 1);
+        const bool fuse = !one_pass(r0) && r0 < n - 1 && !(m < n && r0 == m - 1) && r0 != res_k;
         DDC_TRY(dgemm_trail64(m - r0, n - r0, UX + r0, lda, a.Y + r0, d.ldy, C, lda,
                               fuse ? a.cvec + r0 : nullptr, a.Lpart + r0, d.ldy, 1, st));
         if (fuse) fusedL = (int)ceil_div(m - r0, TRAIL_TILE);

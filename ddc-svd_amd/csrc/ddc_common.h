@@ -114,6 +114,18 @@ void bidiag_plan_f32(ArenaPlan& p, int m, int n, int lda, int upd);
 int bidiag_run_f32(int m, int n, float* A, int lda, double* alpha, double* beta, int upd,
                    Arena& ws, hipStream_t st);
 
+// The column steps from k0 on with the matrix in registers (resident.hip):
+// for what is left of the matrix at k0 >= resident_first(), itself a multiple
+// of align (or -1: never).  *done: steps completed, a multiple of align or
+// min(m, n); less than min(m, n) where the work-groups found no room, A being
+// updated up to there.  Synchronizes st.
+template <typename TS>
+int resident_first(int m, int n, int align);
+void resident_plan(ArenaPlan& p);
+template <typename TS>
+int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int k0, int align,
+                 Arena& ws, hipStream_t st, int* done);
+
 // Mixed-precision SVD of the n x n FP64 matrix A (device pointers): FP32
 // bidiagonalization with update mode upd, FP64 bidiagonal solve, FP32
 // back-transformation, `steps` FP64 refinement steps (separated: the larger
