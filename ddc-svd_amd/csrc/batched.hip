@@ -5,32 +5,40 @@
 // (svd_gpu.c:53).  Method: one-sided (Hestenes) Jacobi by column blocks,
 // one wavefront per matrix.
 //
-//  * A persistent grid of 4-wave workgroups pulls matrix indices from an
-//    atomic counter; the queue is ordered by descending work (n^2 m), so the
-//    large matrices start first and the small ones fill the tail.  A matrix
-//    with min(m, n) >= coop_nt is factored by a whole workgroup (its waves
-//    take disjoint block pairs of each round); from the first smaller matrix
-//    on, every wave takes matrices on its own.
+//  * A persistent grid, one workgroup per CU (8 waves in FP64, 12 in FP32 at
+//    the default variants: all that the registers allow), pulls matrix
+//    indices from an atomic counter; the queue is ordered by descending work
+//    (n^2 m), so the large matrices start first and the small ones fill the
+//    tail.  A matrix with min(m, n) >= coop_nt is factored by a whole
+//    workgroup; from the first smaller matrix on, every wave takes matrices
+//    on its own.  Batches of few large matrices last as long as the largest
+//    one: 256 x 256 takes 18 ms in FP64 (88 before, with four waves).
 //  * A matrix (tall orientation: mt = max(m,n) <= 256 rows, nt = min(m,n)
 //    columns; a wide matrix is processed as its transpose) is split into
-//    column blocks of width B.  For each block pair (I, J) the wave holds the
+//    column blocks of width B.  For each block pair (I, J) a wave holds the
 //    2B columns of the working matrix and of V in registers (lane l holds rows
 //    l, l+64, ...), runs every cross pair (B rounds of B disjoint pairs) and,
-//    on the first visit of a block in a sweep, its internal pairs
-//    (round-robin, B-1 rounds), then writes the columns back.  Only the dot
-//    product gamma needs a wave reduction per rotation: the squared column
-//    norms are reduced when a block pair is loaded and then carried through
-//    the rotations (alpha' = alpha - t gamma, beta' = beta + t gamma).
+//    on the first visit of a block in a sweep, its internal pairs (B-1
+//    rounds).  The rounds are unrolled, so that columns stay in their
+//    registers; the dot products are summed by lane swaps and DPP.  The
+//    squared column norms are reduced once per block pair and then carried
+//    through the rotations (alpha' = alpha - t gamma, beta' = beta + t gamma).
+//  * In FP32, and for a wave alone, block pairs come from memory and go back.
+//    A workgroup takes an FP64 matrix by super-blocks (bj_sweeps_super), one
+//    trip to memory for up to 8 x 8 block pairs.
+//  * FP32 arithmetic (its order, its roundings, its square roots and
+//    divisions) is fixed: vectors of close values show every change of it at
+//    the 1e-5 level.
 //  * Sweeps stop when every pair satisfies |gamma| <= tol sqrt(alpha beta),
 //    tol = sqrt(mt) * eps.  Then sigma_j = ||a_j||, U_j = a_j / sigma_j, and
 //    the columns are written in ascending order of sigma.  Columns of exactly
 //    zero norm are completed to an orthonormal basis by Gram-Schmidt on unit
 //    vectors.
 //
-// Three tunables are picked by measurement (svd_gpu_batched_tune): the kernel
+// Two tunables are picked by measurement (svd_gpu_batched_tune): the kernel
 // variant (block width per row class, which also sets the register budget
-// and so the occupancy), the number of resident workgroups per CU, and the
-// cooperation threshold coop_nt.
+// and so the waves of a workgroup; FP64 only) and the cooperation threshold
+// coop_nt.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -42,12 +50,12 @@
 
 #include "../../include/svd_gpu.h"
 #include "ddc_common.h"
+#include "householder.h"
 
 namespace ddc {
 
 constexpr int BJ_MAXDIM = 256;  // max(m, n) of one matrix
 constexpr int BJ_MAXSWEEP = 40;
-constexpr int BJ_WGW = 4;       // waves per workgroup
 
 struct BatchItem {
   int m, n;
@@ -84,43 +92,133 @@ struct Num<float> {
   static constexpr float big = 1e18f;
 };
 
-// Raw buffer access to one matrix: loads outside [0, count) return 0 and
-// stores there are dropped by the hardware range check, so masked rows and
-// columns need no branches.  Pass idx < 0 for a masked element.
+// Raw buffer access to one column of rows entries (rows = 0: a masked column):
+// loads past it return 0 and stores there are dropped by the hardware range
+// check, so masked rows and columns need no branches, and every column is
+// reached from one lane offset (vo, bytes) and a scalar resource.
 template <typename T>
-struct Buf {
+struct Col {
   __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ Buf(const T* p, int count)
-      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, count * (int)sizeof(T),
+  __device__ __forceinline__ Col(const T* p, int rows)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), 0, rows * (int)sizeof(T),
                                             0x00020000)) {}
-  __device__ __forceinline__ static int off(int idx) {
-    return idx >= 0 ? idx * (int)sizeof(T) : 0x7fffff00;
-  }
-  __device__ __forceinline__ T ld(int idx) const;
-  __device__ __forceinline__ void st(int idx, T v) const;
+  __device__ __forceinline__ T ld(int vo) const;
+  __device__ __forceinline__ void st(int vo, T v) const;
 };
 template <>
-__device__ __forceinline__ double Buf<double>::ld(int idx) const {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off(idx), 0, 0));
+__device__ __forceinline__ double Col<double>::ld(int vo) const {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, 0, 0));
 }
 template <>
-__device__ __forceinline__ float Buf<float>::ld(int idx) const {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off(idx), 0, 0));
+__device__ __forceinline__ float Col<float>::ld(int vo) const {
+  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, vo, 0, 0));
 }
 template <>
-__device__ __forceinline__ void Buf<double>::st(int idx, double v) const {
+__device__ __forceinline__ void Col<double>::st(int vo, double v) const {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(
-      decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0)), v), r, off(idx), 0, 0);
+      decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0, 0, 0)), v), r, vo, 0, 0);
 }
 template <>
-__device__ __forceinline__ void Buf<float>::st(int idx, float v) const {
-  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, off(idx), 0, 0);
+__device__ __forceinline__ void Col<float>::st(int vo, float v) const {
+  __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, vo, 0, 0);
+}
+
+// ---- wave sums without LDS: lane swaps and DPP -----------------------------
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  return dpp_all<CTRL>(v);
+}
+// the value of lane l ^ M (M = 1, 2, 4, 8)
+template <int M, typename T>
+__device__ __forceinline__ T lane_xor(T v) {
+  if constexpr (M == 1) return dpp_mov<DPP_XOR1>(v);
+  if constexpr (M == 2) return dpp_mov<DPP_XOR2>(v);
+  if constexpr (M == 4) return dpp_mov<DPP_HALF_MIRROR>(dpp_mov<DPP_QUAD_REVERSE>(v));
+  if constexpr (M == 8) return dpp_mov<DPP_ROR8>(v);
+}
+template <int W>
+__device__ __forceinline__ void swap_lanes(float& a, float& b) {
+  const unsigned x = __float_as_uint(a), y = __float_as_uint(b);
+  if constexpr (W == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    a = __uint_as_float(l[0]);
+    b = __uint_as_float(l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    a = __uint_as_float(l[0]);
+    b = __uint_as_float(l[1]);
+  }
+}
+// v plus the value of lane l ^ W (W = 16, 32)
+template <int W, typename T>
+__device__ __forceinline__ T add_across(T v) {
+  T a = v, b = v;
+  swap_lanes<W>(a, b);
+  return a + b;
+}
+
+// Wave sum of each g[i], delivered to the 64 / N lanes with lane / (64 / N)
+// == i, summed across lane bits 5, 4, 3, 2, 1, 0 in this order (as
+// reduce_scatter of ddc_common.h, which exchanges through LDS instead).
+// lane_scatter_low: the part after lane bit 5 (of the first N / 2 values).
+template <typename T, int N>
+__device__ __forceinline__ T lane_scatter_low(T (&g)[N]) {
+  static_assert(N == 2 || N == 4 || N == 8 || N == 16, "two to sixteen values");
+  const int lane = threadIdx.x & 63;
+  T v;
+  if constexpr (N >= 4) {
+#pragma unroll
+    for (int j = 0; j < N / 4; ++j) {
+      swap_lanes<16>(g[j], g[j + N / 4]);
+      g[j] += g[j + N / 4];
+    }
+  } else {
+    g[0] = add_across<16>(g[0]);
+  }
+  if constexpr (N >= 8) {
+    const bool up = (lane >> 3) & 1;
+#pragma unroll
+    for (int j = 0; j < N / 8; ++j) {
+      const T lo = g[j], hi = g[j + N / 8];
+      g[j] = (up ? hi : lo) + lane_xor<8>(up ? lo : hi);
+    }
+  } else {
+    g[0] += lane_xor<8>(g[0]);
+  }
+  if constexpr (N >= 16) {
+    const bool up = (lane >> 2) & 1;
+    const T lo = g[0], hi = g[1];
+    v = (up ? hi : lo) + lane_xor<4>(up ? lo : hi);
+  } else {
+    v = g[0] + lane_xor<4>(g[0]);
+  }
+  v += lane_xor<2>(v);
+  v += lane_xor<1>(v);
+  return v;
+}
+template <typename T, int N>
+__device__ __forceinline__ T lane_scatter(T (&g)[N]) {
+#pragma unroll
+  for (int j = 0; j < N / 2; ++j) {
+    swap_lanes<32>(g[j], g[j + N / 2]);
+    g[j] += g[j + N / 2];
+  }
+  return lane_scatter_low<T, N>(g);
 }
 
 template <typename T>
 __device__ __forceinline__ T wsum(T v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  v = add_across<32>(v);
+  v = add_across<16>(v);
+  v += lane_xor<8>(v);
+  v += lane_xor<4>(v);
+  v += lane_xor<2>(v);
+  v += lane_xor<1>(v);
   return v;
 }
 
@@ -158,6 +256,32 @@ __device__ __forceinline__ bool jrot(T al, T be, T ga, T tol, T& c, T& s, T& t, 
   return true;
 }
 
+// In FP64 the square roots and divisions of the general form (about 100
+// dependent instructions) are the longest part of a round.  The tangent only
+// steers convergence, so it comes from the hardware's reciprocals as they are
+// (about 2^-26: the dot product left behind is that factor of the old one);
+// the cosine is brought to full precision, so the rotation is orthogonal to
+// rounding.
+template <>
+__device__ __forceinline__ bool jrot<double>(double al, double be, double ga, double tol,
+                                             double& c, double& s, double& t, double& off) {
+  const double rel = fabs(ga) * __builtin_amdgcn_rsq(al) * __builtin_amdgcn_rsq(be);
+  if (!(al > 0.0) || !(be > 0.0) || !(rel > tol)) return false;
+  off = fmax(off, rel);
+  const double zeta = (be - al) * (0.5 * __builtin_amdgcn_rcp(ga));
+  const double az = fabs(zeta);
+  const double w = fma(az, az, 1.0);
+  const double tm = az > Num<double>::big ? 0.5 * __builtin_amdgcn_rcp(az)
+                                          : __builtin_amdgcn_rcp(az + w * __builtin_amdgcn_rsq(w));
+  t = zeta < 0.0 ? -tm : tm;
+  const double q = fma(t, t, 1.0);
+  const double z = __builtin_amdgcn_rsq(q);
+  const double e = fma(-q * z, z, 1.0);
+  c = fma(z * e, fma(0.375, e, 0.5), z);
+  s = c * t;
+  return true;
+}
+
 // The 2B columns of a block pair held by one wave: positions 0..B-1 are block
 // I, B..2B-1 block J; lane l holds rows l + 64 e.
 template <typename T, int B, int R, int RV>
@@ -182,194 +306,205 @@ __device__ __forceinline__ void rotate_cols(Block<T, B, R, RV>& k, int p, int q,
   }
 }
 
-// Copies column src of block y to column dst of block x (registers).
-template <typename T, int B1, int B2, int R, int RV>
-__device__ __forceinline__ void move_col(Block<T, B1, R, RV>& x, int dst,
-                                         const Block<T, B2, R, RV>& y, int src) {
-#pragma unroll
-  for (int e = 0; e < R; ++e) x.a[dst][e] = y.a[src][e];
-#pragma unroll
-  for (int e = 0; e < RV; ++e) x.v[dst][e] = y.v[src][e];
-}
-template <typename T, int B, int R, int RV>
-__device__ __forceinline__ void move_col(Block<T, B, R, RV>& k, int dst, int src) {
-  move_col(k, dst, k, src);
-}
-
-// Pairs of one round.  Cross rounds (KIND 0) pair position i with B + i;
-// internal rounds (KIND 1) pair, inside each half h, position j with B-1-j
-// (j < B/2): slot i = h * B/2 + j.  Between rounds the positions rotate so
-// that B cross rounds meet every (I, J) pair and B-1 internal rounds every
-// pair inside a block (circle method: position 0 stays, 1..B-1 rotate).
-template <int B, int KIND>
-__host__ __device__ constexpr int pair_p(int i) {
-  return KIND == 0 ? i : (i / (B / 2)) * B + i % (B / 2);
-}
-template <int B, int KIND>
-__host__ __device__ constexpr int pair_q(int i) {
-  return KIND == 0 ? B + i : (i / (B / 2)) * B + B - 1 - i % (B / 2);
-}
-
-// One round: B disjoint rotations.  nrm: lane c holds the squared norm of
-// the column at position c.  The dot products are reduce-scattered across
-// the wave so that the lanes of group i hold pair i's; each group computes
-// its rotation, and the cosines and sines are broadcast.
-template <typename T, int B, int R, int RV, int KIND>
-__device__ __forceinline__ void jround(Block<T, B, R, RV>& k, T& nrm, bool enI, bool enJ, T tol,
-                                       T& off) {
-  const int lane = threadIdx.x & 63;
+// Cross round S of a block pair: B disjoint rotations, column i of block I
+// with column (i + S) mod B of block J.  al, be: the squared norms of the
+// lane's group's pair (group i: the 64 / B lanes from 64 / B i).  The dot
+// products are scattered over the groups; each group computes its rotation,
+// and the cosines and sines are broadcast.  The columns stay where they are
+// (S is a constant); only be moves on by one group.
+template <typename T, int B, int R, int RV, int S>
+__device__ __forceinline__ void cross_round(Block<T, B, R, RV>& k, T& al, T& be, T tol, T& off) {
+  constexpr int GS = 64 / B;
   T g[B];
 #pragma unroll
   for (int i = 0; i < B; ++i) {
-    const bool en = KIND == 0 || (i < B / 2 ? enI : enJ);
     T d = T(0);
-    if (en) {
 #pragma unroll
-      for (int e = 0; e < R; ++e) d += k.a[pair_p<B, KIND>(i)][e] * k.a[pair_q<B, KIND>(i)][e];
+    for (int e = 0; e < R; ++e) d += k.a[i][e] * k.a[B + (i + S) % B][e];
+    g[i] = d;
+  }
+  const T gl = lane_scatter<T, B>(g);
+  T c = T(1), s = T(0), t = T(0);
+  const bool act = jrot(al, be, gl, tol, c, s, t, off);
+  // (the fused forms are spelled out: left to the compiler, a select around
+  // them may split the product from the sum)
+  const T aln = fmax(__builtin_elementwise_fma(-t, gl, al), T(0));
+  const T ben = __builtin_elementwise_fma(t, gl, be);
+  al = act ? aln : al;
+  be = __shfl(act ? ben : be, ((threadIdx.x & 63) + GS) & 63, 64);
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    const T si = rdlane(s, i * GS);
+    if (si != T(0)) rotate_cols(k, i, B + (i + S) % B, rdlane(c, i * GS), si);
+  }
+}
+template <typename T, int B, int R, int RV, int S = 0>
+__device__ __forceinline__ void cross_rounds(Block<T, B, R, RV>& k, T& al, T& be, T tol, T& off) {
+  cross_round<T, B, R, RV, S>(k, al, be, tol, off);
+  if constexpr (S + 1 < B) cross_rounds<T, B, R, RV, S + 1>(k, al, be, tol, off);
+}
+
+// Internal round S (S < B-1) of both halves: half h's columns meet in pairs by
+// the circle method, slot j < B/2 pairing positions j and B-1-j, where
+// position 0 holds column 0 and position x > 0 column 1 + (x-1 + S) mod (B-1).
+// The columns stay where they are.  nrm: lane c holds the squared norm of
+// column c.
+template <int B, int S>
+__host__ __device__ constexpr int circle(int x) {
+  return x == 0 ? 0 : 1 + (x - 1 + S < B - 1 ? x - 1 + S : x - 1 + S - (B - 1));
+}
+template <typename T, int B, int R, int RV, int S>
+__device__ __forceinline__ void intra_round(Block<T, B, R, RV>& k, T& nrm, bool enI, bool enJ,
+                                            T tol, T& off) {
+  const int lane = threadIdx.x & 63;
+  constexpr int GS = 64 / B, H = B / 2;  // lanes per pair, pairs per half
+  T g[B];
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    T d = T(0);
+    if (i < H ? enI : enJ) {
+#pragma unroll
+      for (int e = 0; e < R; ++e)
+        d += k.a[i / H * B + circle<B, S>(i % H)][e] *
+             k.a[i / H * B + circle<B, S>(B - 1 - i % H)][e];
     }
     g[i] = d;
   }
-  constexpr int GS = 64 / B;  // lanes per group
-  const T gl = reduce_scatter<T, B>(g);
-  const int li = lane / GS;  // the pair this lane's group handles
-  const int pl = KIND == 0 ? li : (li / (B / 2)) * B + li % (B / 2);
-  const int ql = KIND == 0 ? B + li : (li / (B / 2)) * B + B - 1 - li % (B / 2);
-  const T al = __shfl(nrm, pl, 64), be = __shfl(nrm, ql, 64);
+  const T gl = lane_scatter<T, B>(g);
+  const int h = lane / GS / H, j = lane / GS % H;  // the pair this lane's group handles
+  const T al = __shfl(nrm, h * B + circle<B, S>(j), 64);
+  const T be = __shfl(nrm, h * B + circle<B, S>(B - 1 - j), 64);
   T c = T(1), s = T(0), t = T(0);
   const bool act = jrot(al, be, gl, tol, c, s, t, off);
-  const T aln = act ? fmax(al - t * gl, T(0)) : al;
-  const T ben = act ? be + t * gl : be;
-  // new norms back to the column lanes
-  int slot;
-  bool qside;
-  if (KIND == 0) {
-    qside = lane >= B;
-    slot = qside ? lane - B : lane;
-  } else {
-    const int h = lane / B, x = lane % B;
-    qside = x >= B / 2;
-    slot = h * (B / 2) + (qside ? B - 1 - x : x);
-  }
-  slot = lane < 2 * B ? slot : 0;
+  const T aln = act ? fmax(__builtin_elementwise_fma(-t, gl, al), T(0)) : al;
+  const T ben = act ? __builtin_elementwise_fma(t, gl, be) : be;
+  // new norms back to the column lanes: column x is at position pos
+  const int x = lane % B, y = x - 1 - S;
+  const int pos = x == 0 ? 0 : 1 + (y < 0 ? y + B - 1 : y);
+  const bool qside = pos >= H;
+  const int slot = lane < 2 * B ? lane / B * H + (qside ? B - 1 - pos : pos) : 0;
   const T np = __shfl(aln, slot * GS, 64), nq = __shfl(ben, slot * GS, 64);
   if (lane < 2 * B) nrm = qside ? nq : np;
 #pragma unroll
   for (int i = 0; i < B; ++i) {
     const T si = rdlane(s, i * GS);
     if (si != T(0))
-      rotate_cols(k, pair_p<B, KIND>(i), pair_q<B, KIND>(i), rdlane(c, i * GS), si);
+      rotate_cols(k, i / H * B + circle<B, S>(i % H), i / H * B + circle<B, S>(B - 1 - i % H),
+                  rdlane(c, i * GS), si);
+  }
+}
+template <typename T, int B, int R, int RV, int S = 0>
+__device__ __forceinline__ void intra_rounds(Block<T, B, R, RV>& k, T& nrm, bool enI, bool enJ,
+                                             T tol, T& off) {
+  intra_round<T, B, R, RV, S>(k, nrm, enI, enJ, tol, off);
+  if constexpr (S + 2 < B) intra_rounds<T, B, R, RV, S + 1>(k, nrm, enI, enJ, tol, off);
+}
+
+// Half H (0: block I, 1: block J) of a block pair from and to memory: the
+// columns from c0 on (c0 < 0, or past nt: masked).
+template <int H, typename T, int B, int R, int RV>
+__device__ __forceinline__ void load_half(Block<T, B, R, RV>& k, const T* W, const T* WV, int mt,
+                                          int nt, int c0) {
+  const int vo = (threadIdx.x & 63) * (int)sizeof(T);
+  constexpr int STEP = 64 * (int)sizeof(T);
+#pragma unroll
+  for (int c = 0; c < B; ++c) {
+    const bool ok = c0 >= 0 && c0 + c < nt;
+    const int cc = ok ? c0 + c : 0;
+    const Col<T> ca(W + (int64_t)cc * mt, ok ? mt : 0), cv(WV + (int64_t)cc * nt, ok ? nt : 0);
+#pragma unroll
+    for (int e = 0; e < R; ++e) k.a[H * B + c][e] = ca.ld(vo + e * STEP);
+#pragma unroll
+    for (int e = 0; e < RV; ++e) k.v[H * B + c][e] = cv.ld(vo + e * STEP);
+  }
+}
+template <int H, typename T, int B, int R, int RV>
+__device__ __forceinline__ void store_half(const Block<T, B, R, RV>& k, T* W, T* WV, int mt, int nt,
+                                           int c0) {
+  const int vo = (threadIdx.x & 63) * (int)sizeof(T);
+  constexpr int STEP = 64 * (int)sizeof(T);
+  // the column resources are made anew here instead of being kept through
+  // the rounds
+  asm volatile("" : "+s"(c0), "+s"(mt), "+s"(nt));
+#pragma unroll
+  for (int c = 0; c < B; ++c) {
+    const bool ok = c0 >= 0 && c0 + c < nt;
+    const int cc = ok ? c0 + c : 0;
+    const Col<T> ca(W + (int64_t)cc * mt, ok ? mt : 0), cv(WV + (int64_t)cc * nt, ok ? nt : 0);
+#pragma unroll
+    for (int e = 0; e < R; ++e) ca.st(vo + e * STEP, k.a[H * B + c][e]);
+#pragma unroll
+    for (int e = 0; e < RV; ++e) cv.st(vo + e * STEP, k.v[H * B + c][e]);
   }
 }
 
-// Position rotations between rounds (registers and norms).
+// Squared norms of the columns held: column c's on the 32 / B lanes from
+// (32 / B) c.
 template <typename T, int B, int R, int RV>
-__device__ __forceinline__ void shift_cross(Block<T, B, R, RV>& k, T& nrm) {
-  const int lane = threadIdx.x & 63;
-  Block<T, 1, R, RV> tmp;
-  move_col(tmp, 0, k, B);
+__device__ __forceinline__ T col_norms(const Block<T, B, R, RV>& k) {
+  T part[2 * B];
+  if constexpr (R == 1) {
+    // one entry per lane: the squares of lanes l and l + 32 in one fused
+    // multiply-add
 #pragma unroll
-  for (int x = 0; x < B - 1; ++x) move_col(k, B + x, B + x + 1);
-  move_col(k, 2 * B - 1, tmp, 0);
-  const int src = (lane >= B && lane < 2 * B) ? B + (lane - B + 1) % B : lane;
-  nrm = __shfl(nrm, src, 64);
-}
-
-template <typename T, int B, int R, int RV>
-__device__ __forceinline__ void shift_intra(Block<T, B, R, RV>& k, T& nrm) {
-  const int lane = threadIdx.x & 63;
+    for (int c = 0; c < B; ++c) {
+      T x = k.a[c][0], y = k.a[B + c][0];
+      swap_lanes<32>(x, y);
+      part[c] = __builtin_elementwise_fma(x, x, y * y);
+    }
+    return lane_scatter_low<T, 2 * B>(part);
+  } else {
 #pragma unroll
-  for (int h = 0; h < 2 * B; h += B) {
-    Block<T, 1, R, RV> tmp;
-    move_col(tmp, 0, k, h + 1);
+    for (int c = 0; c < 2 * B; ++c) {
+      T s = T(0);
 #pragma unroll
-    for (int x = 1; x < B - 1; ++x) move_col(k, h + x, h + x + 1);
-    move_col(k, h + B - 1, tmp, 0);
+      for (int e = 0; e < R; ++e) s += k.a[c][e] * k.a[c][e];
+      part[c] = s;
+    }
+    return lane_scatter<T, 2 * B>(part);
   }
-  const int x = lane % B;
-  const int src = (lane < 2 * B && x >= 1) ? lane - x + 1 + x % (B - 1) : lane;
-  nrm = __shfl(nrm, src, 64);
 }
 
 // One block-pair step.  cI / cJ: first columns of the blocks (cJ < 0: block I
-// alone).  Returns the largest relative dot product seen.
+// alone).  Returns the largest relative dot product seen by the lane.
 template <typename T, int B, int R, int RV>
-__device__ __forceinline__ T block_step(T* __restrict__ W, T* __restrict__ WV, int mt, int nt, int cI, int cJ,
-                        bool intraI, bool intraJ, T tol) {
+__device__ __forceinline__ T block_step(T* __restrict__ W, T* __restrict__ WV, int mt, int nt,
+                                        int cI, int cJ, bool intraI, bool intraJ, T tol) {
   const int lane = threadIdx.x & 63;
-  const Buf<T> bw(W, mt * nt), bv(WV, nt * nt);
+  cI = __builtin_amdgcn_readfirstlane(cI);
+  cJ = __builtin_amdgcn_readfirstlane(cJ);
   Block<T, B, R, RV> k;
-  T part[2 * B];
-#pragma unroll
-  for (int c = 0; c < 2 * B; ++c) {
-    const int col = c < B ? cI + c : cJ + (c - B);
-    const bool ok = (c < B || cJ >= 0) && col < nt;
-#pragma unroll
-    for (int e = 0; e < R; ++e) {
-      const int r = lane + 64 * e;
-      k.a[c][e] = bw.ld(ok && r < mt ? r + col * mt : -1);
-    }
-#pragma unroll
-    for (int e = 0; e < RV; ++e) {
-      const int r = lane + 64 * e;
-      k.v[c][e] = bv.ld(ok && r < nt ? r + col * nt : -1);
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 2 * B; ++c) {
-    T s = T(0);
-#pragma unroll
-    for (int e = 0; e < R; ++e) s += k.a[c][e] * k.a[c][e];
-    part[c] = s;
-  }
-  T nrm = T(0);
-#pragma unroll
-  for (int c = 0; c < 2 * B; ++c) {
-    const T sc = wsum(part[c]);
-    nrm = lane == c ? sc : nrm;
-  }
-
+  load_half<0>(k, W, WV, mt, nt, cI);
+  load_half<1>(k, W, WV, mt, nt, cJ);
+  constexpr int GN = 32 / B, GS = 64 / B;  // lanes per column, per pair
+  T nrm = col_norms(k);
   T off = T(0);
+  T al, be;
   if (intraI || intraJ) {
-#pragma unroll 1
-    for (int r = 0; r < B - 1; ++r) {
-      jround<T, B, R, RV, 1>(k, nrm, intraI, intraJ, tol, off);
-      shift_intra(k, nrm);
-    }
+    nrm = __shfl(nrm, (lane & (2 * B - 1)) * GN, 64);
+    intra_rounds(k, nrm, intraI, intraJ, tol, off);
+    al = __shfl(nrm, lane / GS, 64);
+    be = __shfl(nrm, B + lane / GS, 64);
+  } else {
+    al = __shfl(nrm, lane / GS * GN, 64);
+    be = __shfl(nrm, (B + lane / GS) * GN, 64);
   }
-  if (cJ >= 0) {
-#pragma unroll 1
-    for (int r = 0; r < B; ++r) {
-      jround<T, B, R, RV, 0>(k, nrm, true, true, tol, off);
-      shift_cross(k, nrm);
-    }
-  }
-  // recompute the store addresses here instead of keeping the load
-  // addresses live through the rounds
-  asm volatile("" : "+v"(cI), "+v"(cJ), "+v"(mt), "+v"(nt));
-#pragma unroll
-  for (int c = 0; c < 2 * B; ++c) {
-    const int col = c < B ? cI + c : cJ + (c - B);
-    const bool ok = (c < B || cJ >= 0) && col < nt;
-#pragma unroll
-    for (int e = 0; e < R; ++e) {
-      const int r = lane + 64 * e;
-      bw.st(ok && r < mt ? r + col * mt : -1, k.a[c][e]);
-    }
-#pragma unroll
-    for (int e = 0; e < RV; ++e) {
-      const int r = lane + 64 * e;
-      bv.st(ok && r < nt ? r + col * nt : -1, k.v[c][e]);
-    }
-  }
-  return wmax(off);
+  if (cJ >= 0) cross_rounds(k, al, be, tol, off);
+  store_half<0>(k, W, WV, mt, nt, cI);
+  store_half<1>(k, W, WV, mt, nt, cJ);
+  return off;
 }
 
 // Pair i of round r of the round-robin schedule of P players (circle method):
 // every pair of 0..P-1 (P even) appears once in rounds 0..P-2.
+// (r < P - 1 and i < P / 2: the remainder by P - 1 is one subtraction)
+__host__ __device__ constexpr int rr_mod(int P, int x) { return x >= P - 1 ? x - (P - 1) : x; }
 __host__ __device__ constexpr int rr_p(int P, int r, int i) {
-  return i == 0 ? 0 : 1 + (i - 1 + r) % (P - 1);
+  return i == 0 ? 0 : 1 + rr_mod(P, i - 1 + r);
 }
-__host__ __device__ constexpr int rr_q(int P, int r, int i) { return 1 + (P - 2 - i + r) % (P - 1); }
+__host__ __device__ constexpr int rr_q(int P, int r, int i) {
+  return 1 + rr_mod(P, P - 2 - i + r);
+}
 
 // A team: the nw waves of a workgroup that factor one matrix together
 // (nw = 1: a wave alone).  w is the wave's index in the team.
@@ -405,12 +540,15 @@ __device__ __forceinline__ T team_max(T v, Team t, T* red) {
 template <typename T, int B, int R, int RV>
 __device__ __forceinline__ int bj_sweeps(T* W, T* WV, int mt, int nt, Team t, T* red) {
   const T tol = Num<T>::eps * sqrt(T(mt));
+  mt = __builtin_amdgcn_readfirstlane(mt);
+  nt = __builtin_amdgcn_readfirstlane(nt);
   const int nb = (nt + B - 1) / B;
   const int nbe = nb + (nb & 1);
+  const int w = __builtin_amdgcn_readfirstlane(t.w), nw = __builtin_amdgcn_readfirstlane(t.nw);
   for (int sw = 0; sw < BJ_MAXSWEEP; ++sw) {
     T off = T(0);
     for (int r = 0; r < nbe - 1; ++r) {
-      for (int i = t.w; i < nbe / 2; i += t.nw) {
+      for (int i = w; i < nbe / 2; i += nw) {
         int I = rr_p(nbe, r, i), J = rr_q(nbe, r, i);
         if (I > J) {
           const int x = I;
@@ -422,6 +560,91 @@ __device__ __forceinline__ int bj_sweeps(T* W, T* WV, int mt, int nt, Team t, T*
         off = fmax(off, block_step<T, B, R, RV>(W, WV, mt, nt, I * B, alone ? -1 : J * B, r == 0,
                                                 r == 0 && !alone, tol));
       }
+      t.sync();
+    }
+    off = team_max(off, t, red);
+    if (!(off > tol)) return sw + 1;
+  }
+  return -1;
+}
+
+// The sweeps of one FP64 matrix by a whole workgroup (nw waves).  Taking each
+// block pair from memory and back, as above, moves the matrix and V through
+// L2 and the Infinity Cache once per round: 16 B (m + n) per rotation and
+// column pair at B = 4, 3.9 TB/s over a batch of 10,000, and each round waits
+// for it.  Here the column blocks are grouped by q <= nw into super-blocks.
+//  * Pairs inside the super-blocks: as above, all super-blocks side by side.
+//  * Pairs across super-blocks S < T: wave w holds block w of S in registers
+//    while every T passes by; block w of T, then its successors, come from
+//    the neighbouring wave through LDS, so all q x q pairs are met with one
+//    trip to memory for T (and one per S for all T).
+// xch: 64 B (R + RV) values per wave.
+template <typename T, int B, int R, int RV>
+__device__ __forceinline__ int bj_sweeps_super(T* W, T* WV, int mt, int nt, Team t, T* red,
+                                               T* xch) {
+  const T tol = Num<T>::eps * sqrt(T(mt));
+  const int lane = threadIdx.x & 63;
+  mt = __builtin_amdgcn_readfirstlane(mt);
+  nt = __builtin_amdgcn_readfirstlane(nt);
+  const int w = __builtin_amdgcn_readfirstlane(t.w), nw = __builtin_amdgcn_readfirstlane(t.nw);
+  const int nb = (nt + B - 1) / B;
+  const int ns = (nb + nw - 1) / nw, q = (nb + ns - 1) / ns;
+  const int qe = q + (q & 1), hq = qe / 2;
+  constexpr int HW = B * (R + RV) * 64;  // values of half a block pair
+  constexpr int GN = 32 / B, GS = 64 / B;
+  const int next = w + 1 < q ? w + 1 : 0;
+  for (int sw = 0; sw < BJ_MAXSWEEP; ++sw) {
+    T off = T(0);
+    for (int r = 0; r < max(qe - 1, 1); ++r) {
+      for (int i = w; i < ns * hq; i += nw) {
+        const int s = i / hq, pi = i - s * hq;
+        const int x = rr_p(qe, r, pi), y = rr_q(qe, r, pi);
+        const int lo = min(x, y), hi = max(x, y);
+        const int I = s * q + lo, J = s * q + hi;
+        const bool alone = hi >= q || J >= nb;
+        if (I >= nb || (alone && r != 0)) continue;
+        off = fmax(off, block_step<T, B, R, RV>(W, WV, mt, nt, I * B, alone ? -1 : J * B, r == 0,
+                                                r == 0 && !alone, tol));
+      }
+      t.sync();
+    }
+    // (waves past q go along with masked columns: branches around parts of
+    // the loops would cost the others copies of all their columns)
+    for (int S = 0; S + 1 < ns; ++S) {
+      Block<T, B, R, RV> k;
+      load_half<0>(k, W, WV, mt, nt, w < q ? (S * q + w) * B : -1);
+      for (int U = S + 1; U < ns; ++U) {
+        load_half<1>(k, W, WV, mt, nt, w < q ? (U * q + w) * B : -1);
+#pragma unroll 1
+        for (int r = 0;;) {
+          const T nrm = col_norms(k);
+          T al = __shfl(nrm, lane / GS * GN, 64), be = __shfl(nrm, (B + lane / GS) * GN, 64);
+          cross_rounds(k, al, be, tol, off);
+          if (++r == q) break;
+#pragma unroll
+          for (int c = 0; c < B; ++c) {
+            T* to = xch + w * HW + c * (R + RV) * 64 + lane;
+#pragma unroll
+            for (int e = 0; e < R; ++e) to[e * 64] = k.a[B + c][e];
+#pragma unroll
+            for (int e = 0; e < RV; ++e) to[(R + e) * 64] = k.v[B + c][e];
+          }
+          __syncthreads();
+#pragma unroll
+          for (int c = 0; c < B; ++c) {
+            const T* from = xch + next * HW + c * (R + RV) * 64 + lane;
+#pragma unroll
+            for (int e = 0; e < R; ++e) k.a[B + c][e] = from[e * 64];
+#pragma unroll
+            for (int e = 0; e < RV; ++e) k.v[B + c][e] = from[(R + e) * 64];
+          }
+          __syncthreads();
+        }
+        // block w + q - 1 (mod q) of U is here now
+        store_half<1>(k, W, WV, mt, nt, w < q ? (U * q + (w > 0 ? w - 1 : q - 1)) * B : -1);
+        t.sync();
+      }
+      store_half<0>(k, W, WV, mt, nt, w < q ? (S * q + w) * B : -1);
       t.sync();
     }
     off = team_max(off, t, red);
@@ -546,22 +769,26 @@ __device__ void bj_finish(const BatchItem& it, const BjArgs<T>& g, T* W, T* WV, 
   t.sync();
 }
 
-template <typename T, int B, int R, int RV>
-__device__ __forceinline__ void bj_matrix(const BatchItem& it, const BjArgs<T>& g, int k,
-                                          Team t, T* sig, int* rk, T* red) {
-  const int mt = it.m > it.n ? it.m : it.n, nt = it.m > it.n ? it.n : it.m;
-  T* W = g.W + it.wa;
-  T* WV = g.WV + it.wv;
-  const T scale = bj_load(it, g.A, W, WV, mt, nt, t, red);
-  const int sweeps = bj_sweeps<T, B, R, RV>(W, WV, mt, nt, t, red);
-  bj_finish(it, g, W, WV, mt, nt, scale, sig, rk, t);
-  if (g.info && threadIdx.x % (64 * t.nw) == 0) g.info[k] = sweeps;
-}
-
 __device__ __forceinline__ int64_t uni64(int64_t x) {
   const int lo = __builtin_amdgcn_readfirstlane((int)(x & 0xffffffffll));
   const int hi = __builtin_amdgcn_readfirstlane((int)(x >> 32));
   return ((int64_t)hi << 32) | (int64_t)(unsigned)lo;
+}
+
+template <typename T, int B, int R, int RV>
+__device__ __forceinline__ void bj_matrix(const BatchItem& it, const BjArgs<T>& g, int k,
+                                          Team t, T* sig, int* rk, T* red, T* xch) {
+  const int mt = it.m > it.n ? it.m : it.n, nt = it.m > it.n ? it.n : it.m;
+  T* W = (T*)uni64((int64_t)(g.W + it.wa));
+  T* WV = (T*)uni64((int64_t)(g.WV + it.wv));
+  const T scale = bj_load(it, g.A, W, WV, mt, nt, t, red);
+  int sweeps;
+  if (sizeof(T) == 8 && t.nw > 1)
+    sweeps = bj_sweeps_super<T, B, R, RV>(W, WV, mt, nt, t, red, xch);
+  else
+    sweeps = bj_sweeps<T, B, R, RV>(W, WV, mt, nt, t, red);
+  bj_finish(it, g, W, WV, mt, nt, scale, sig, rk, t);
+  if (g.info && threadIdx.x % (64 * t.nw) == 0) g.info[k] = sweeps;
 }
 
 // The descriptor as wave-uniform (scalar) values.
@@ -584,20 +811,25 @@ __device__ __forceinline__ int pop_wave(int* counter) {
   return __builtin_amdgcn_readfirstlane(idx);
 }
 
-// Persistent kernel, BJ_WGW waves per workgroup.  While the queue head holds
+// Persistent kernel, one workgroup per CU.  While the queue head holds
 // matrices with min(m, n) >= coop_nt, the workgroup's waves factor each one
 // together; from the first smaller matrix on (the queue is sorted by work)
 // every wave takes matrices on its own.
 // B12 / B34: block width for matrices with up to 128 / up to 256 rows.
 // MINW: resident waves per SIMD the register allocation must allow.
 template <typename T, int B12, int B34, int MINW>
-__global__ __launch_bounds__(64 * BJ_WGW, MINW) void bj_kernel(BjArgs<T> g) {
-  __shared__ T sig[BJ_WGW][BJ_MAXDIM];
-  __shared__ int rk[BJ_WGW][BJ_MAXDIM];
-  __shared__ T red[BJ_WGW];
+__global__ __launch_bounds__(256 * MINW, MINW) void bj_kernel(BjArgs<T> g) {
+  constexpr int WGW = 4 * MINW;  // waves per workgroup: all that a CU holds
+  __shared__ T sig[WGW][BJ_MAXDIM];
+  __shared__ int rk[WGW][BJ_MAXDIM];
+  __shared__ T red[WGW];
+  // bj_sweeps_super: at most 2 + 2 values per lane and column up to 128 rows,
+  // 4 + 4 beyond
+  constexpr int XW = sizeof(T) == 8 ? 64 * (B12 * 4 > B34 * 8 ? B12 * 4 : B34 * 8) : 1;
+  __shared__ T xch[WGW * XW];
   __shared__ int s_idx;
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  Team t{w, BJ_WGW};
+  Team t{w, WGW};
   bool coop = true;
   for (;;) {
     int idx;
@@ -629,7 +861,7 @@ __global__ __launch_bounds__(64 * BJ_WGW, MINW) void bj_kernel(BjArgs<T> g) {
     const int R = (mt + 63) / 64, RV = (nt + 63) / 64;
 #define BJ_CASE(R_, RV_)                                                  \
   if (R == R_ && RV == RV_) {                                             \
-    bj_matrix<T, (R_ <= 2 ? B12 : B34), R_, RV_>(it, g, k, t, sg, rkk, rd); \
+    bj_matrix<T, (R_ <= 2 ? B12 : B34), R_, RV_>(it, g, k, t, sg, rkk, rd, xch); \
     continue;                                                             \
   }
     BJ_CASE(1, 1)
@@ -657,12 +889,13 @@ __global__ void k_fill_i32(int* p, int v, int n) {
 
 struct BjVariant {
   int b12, b34;
+  int w64, w32;  // waves per SIMD
   const void* f64;
   const void* f32;
 };
 
 #define BJ_VARIANT(B12, B34, W64, W32) \
-  {B12, B34, (const void*)&bj_kernel<double, B12, B34, W64>, \
+  {B12, B34, W64, W32, (const void*)&bj_kernel<double, B12, B34, W64>, \
    (const void*)&bj_kernel<float, B12, B34, W32>}
 static const BjVariant kVariants[] = {
     BJ_VARIANT(8, 4, 2, 3),
@@ -672,9 +905,10 @@ static const BjVariant kVariants[] = {
 };
 #undef BJ_VARIANT
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
-static const int kWgsPerCu[] = {2, 3};
+static const int kWgsPerCu[] = {1};
+// (one workgroup holds all the waves a CU can)
 // first entry: the threshold used while the variants are compared
-static const int kCoopNt[] = {32, 1, 8, 16, 64, BJ_MAXDIM + 1};
+static const int kCoopNt[] = {32, 1, 8, 16, 64, 96, 128, 192, BJ_MAXDIM + 1};
 
 // A launch configuration: kernel variant, resident workgroups per CU, and
 // the smallest min(m, n) a whole workgroup factors together.
@@ -687,8 +921,9 @@ static int bj_launch(const BjConfig& c, int cus, BjArgs<T> a, hipStream_t st) {
   const BjVariant& v = kVariants[c.variant];
   const void* f = sizeof(T) == 8 ? v.f64 : v.f32;
   a.coop_nt = c.coop_nt;
+  const int threads = 256 * (sizeof(T) == 8 ? v.w64 : v.w32);
   void* params[] = {&a};
-  DDC_HIP(hipLaunchKernel(f, dim3(cus * c.wgs), dim3(64 * BJ_WGW), params, 0, st));
+  DDC_HIP(hipLaunchKernel(f, dim3(cus * c.wgs), dim3(threads), params, 0, st));
   return DDC_OK;
 }
 
@@ -770,8 +1005,26 @@ static int bj_time(svd_gpu_batch* p, const BjConfig& c, const void* dA, void* dS
   return DDC_OK;
 }
 
-// The autotuner: times (variant, workgroups per CU) with a middle
-// cooperation threshold, then the thresholds for the best pair, each on the
+// The variant of an FP32 batch, by its sizes: the results depend on the block
+// width in their last digits, and the two widths that come into question are
+// within 2% of each other wherever the largest matrix decides the time, so a
+// timing would pick one or the other from run to run.  Blocks of 4 throughout
+// are the faster ones (by 2%: 17.9 against 18.3 ms for 2,500 matrices up to
+// 256) for batches that are mostly a few matrices above 224 rows; blocks of 8
+// up to 128 rows everywhere else (13.1 against 17.0 ms for 10,000 up to 128).
+static int bj_variant_f32(const svd_gpu_batch* p) {
+  int rows = 0;
+  double most = 0.0;
+  for (int k = 0; k < p->count; ++k) {
+    const int mt = std::max(p->m[k], p->n[k]), nt = std::min(p->m[k], p->n[k]);
+    rows = std::max(rows, mt);
+    most = std::max(most, (double)nt * nt * mt);
+  }
+  return rows > 224 && p->work < 350.0 * most ? 1 : 0;
+}
+
+// The autotuner: times the variants (FP64; see bj_variant_f32) with a middle
+// cooperation threshold, then the thresholds for the best one, each on the
 // whole batch.  (A half-size sample was tried: it keeps the largest
 // matrices, whose latency floors the makespan, but only half of the bulk,
 // and ranked configurations 25% apart in the wrong order.)
@@ -786,8 +1039,10 @@ static int bj_tune(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* d
   float best = 1e30f;
   BjConfig bc;
   int rc = DDC_OK;
+  const int only = p->dtype == SVD_GPU_F32 ? bj_variant_f32(p) : -1;
   for (int v = 0; v < kNumVariants && !rc; ++v)
     for (int wg : kWgsPerCu) {
+      if (only >= 0 && v != only) continue;
       BjConfig c;
       c.variant = v;
       c.wgs = wg;
@@ -920,7 +1175,10 @@ static int bj_plan(svd_gpu_batch* p, int count, const int* m, const int* n, int 
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto f = g_tune_cache.find(tune_key(p));
-    if (f != g_tune_cache.end()) p->cfg = f->second;
+    if (f != g_tune_cache.end()) {
+      p->cfg = f->second;
+      if (dtype == SVD_GPU_F32) p->cfg.variant = bj_variant_f32(p);
+    }
   }
   return DDC_OK;
 }
@@ -967,9 +1225,9 @@ static int bj_run(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* dV
 constexpr size_t BJ_NA_BYTES = (size_t)32 << 20;  // device scratch per GPU
 constexpr int BJ_NA_MAXCOUNT = 4096;              // matrices per call
 constexpr int BJ_NA_MAXDEV = 64;
-// fixed launch configuration: variant 1 (column blocks of 4), two resident
-// workgroups per CU, whole-workgroup factorization from min(m, n) = 32 on
-static const BjConfig kNoallocConfig = {1, 2, 32};
+// fixed launch configuration: variant 1 (column blocks of 4), one workgroup
+// per CU, whole-workgroup factorization from min(m, n) = 32 on
+static const BjConfig kNoallocConfig = {1, 1, 32};
 
 static __device__ __align__(256) char scratch[BJ_NA_BYTES];
 

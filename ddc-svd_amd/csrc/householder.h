@@ -55,6 +55,7 @@ __device__ __forceinline__ double dpp_all(double v) {
 }
 constexpr int DPP_XOR1 = 0xB1;          // quad_perm [1,0,3,2]
 constexpr int DPP_XOR2 = 0x4E;          // quad_perm [2,3,0,1]
+constexpr int DPP_QUAD_REVERSE = 0x1B;  // quad_perm [3,2,1,0]
 constexpr int DPP_HALF_MIRROR = 0x141;  // lane i of eight from lane 7 - i
 constexpr int DPP_MIRROR = 0x140;       // lane i of sixteen from lane 15 - i
 constexpr int DPP_ROR8 = 0x128;         // rows of sixteen rotated by eight

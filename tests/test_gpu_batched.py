@@ -172,3 +172,29 @@ def test_batched_rejects_bad_shapes(ddcsvd):
         BatchedSvd([300], [10])
     with pytest.raises(ddcsvd.SvdGpuError):
         BatchedSvd([10, 0], [10, 5])
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+def test_batched_block_edges(ddcsvd, dtype, variant):
+    """Column counts around multiples of the column blocks (2, 4, 8) and of the
+    super-blocks of a whole workgroup (8 or 12 blocks), row counts around the
+    register classes (64 rows each); all matrices by whole workgroups, then
+    all by single waves."""
+    from ddcsvd import batched
+    gpu_case(f"batched block edges {dtype} variant {variant}")
+    ns = [1, 2, 7, 8, 9, 31, 32, 33, 47, 48, 49, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161,
+          193, 255, 256]
+    ms = [n + d if n + d <= 256 else n for n, d in zip(ns, [0, 62, 57, 120, 0, 33, 0, 1, 80, 16, 15,
+                                                          1, 0, 63, 33, 0, 95, 1, 0, 0, 32, 31, 63,
+                                                          1, 0])]
+    ms[6::9], ns[6::9] = ns[6::9], ms[6::9]  # some of them wide
+    b = batched.BatchedSvd(ms, ns, dtype=dtype)
+    mats = _mats(ms, ns, seed=11)
+    A = b.pack(mats)
+    for coop in (1, 257):
+        b.set_config(variant, 1, coop)
+        S, U, V = b.outputs()
+        b.run(A, S, U, V)
+        _check_batch(b, mats, S, U, V, dtype)
+    b.close()
