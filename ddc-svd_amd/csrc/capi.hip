@@ -42,6 +42,7 @@ struct Ctx {
   // pinned staging buffers of the host-buffer entry points, the events of
   // the copies that last used them and whether those may still be running
   char* stage[2] = {nullptr, nullptr};
+  size_t stage_cap = 0;  // bytes of each
   hipEvent_t sev[2] = {nullptr, nullptr};
   bool spend[2] = {false, false};
 } g_ctx;
@@ -171,28 +172,43 @@ static int arena_get(size_t bytes, Arena& ws, hipStream_t st) {
 // ---- host <-> device copies of the host-buffer entry points ----------------
 // A copy from or to pageable memory goes through two pinned staging buffers:
 // the CPU copies one slice between the caller's buffer and a staging buffer
-// while the DMA engine moves the other (a pageable hipMemcpy stages through
-// the runtime's own buffers at a fraction of the link's rate).
+// while the DMA engine moves the other.  A pageable hipMemcpy2D with a pitch
+// moves its columns one by one, which was most of a small call: svd_gpu of
+// 640 x 480 takes 3.9 ms (17.7 with direct copies), of 96 x 64 1.15 (2.9),
+// bidiag_gpu of 2048 x 1536 8.9 (33.3), of 640 x 480 2.0 (9.6).
 
-constexpr size_t STAGE_BYTES = size_t(32) << 20;  // per staging buffer
-constexpr size_t STAGE_MIN = size_t(4) << 20;     // smaller copies go directly
-
-static int stage_init() {
-  if (g_ctx.stage[1]) return DDC_OK;
-  for (int b = 0; b < 2; ++b) {
-    if (!g_ctx.sev[b]) DDC_HIP(hipEventCreateWithFlags(&g_ctx.sev[b], hipEventDisableTiming));
-    if (!g_ctx.stage[b])
-      DDC_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_ctx.stage[b]), STAGE_BYTES,
-                            hipHostMallocDefault));
-  }
-  return DDC_OK;
-}
+constexpr size_t STAGE_BYTES = size_t(32) << 20;  // per staging buffer, at most
+constexpr size_t STAGE_SLICE = size_t(1) << 20;   // slices of a copy, at least
 
 static int stage_wait(int b) {
   if (g_ctx.spend[b]) {
     DDC_HIP(hipEventSynchronize(g_ctx.sev[b]));
     g_ctx.spend[b] = false;
   }
+  return DDC_OK;
+}
+
+// Bytes per slice of a copy of `bytes` (columns of width bytes): a third of
+// it, so that the CPU's copies and the DMA overlap, between STAGE_SLICE and
+// STAGE_BYTES.
+static size_t stage_slice(size_t bytes, size_t width) {
+  return std::min(STAGE_BYTES, std::max({STAGE_SLICE, width, bytes / 3}));
+}
+
+// two buffers of at least slice bytes
+static int stage_init(size_t slice) {
+  if (g_ctx.stage_cap >= slice) return DDC_OK;
+  size_t cap = STAGE_SLICE;
+  while (cap < slice) cap *= 2;
+  g_ctx.stage_cap = 0;
+  for (int b = 0; b < 2; ++b) {
+    DDC_TRY(stage_wait(b));
+    if (!g_ctx.sev[b]) DDC_HIP(hipEventCreateWithFlags(&g_ctx.sev[b], hipEventDisableTiming));
+    if (g_ctx.stage[b]) DDC_HIP(hipHostFree(g_ctx.stage[b]));
+    g_ctx.stage[b] = nullptr;
+    DDC_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_ctx.stage[b]), cap, hipHostMallocDefault));
+  }
+  g_ctx.stage_cap = cap;
   return DDC_OK;
 }
 
@@ -247,12 +263,13 @@ static void host_copy2d(char* dst, size_t dpitch, const char* src, size_t spitch
 // host (pageable) -> device, stream-ordered on st; the caller synchronizes
 static int copy_h2d(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width,
                     size_t cols, hipStream_t st) {
-  if (width * cols < STAGE_MIN || width > STAGE_BYTES) {
+  if (width > STAGE_BYTES) {
     DDC_HIP(hipMemcpy2DAsync(dst, dpitch, src, spitch, width, cols, hipMemcpyHostToDevice, st));
     return DDC_OK;
   }
-  DDC_TRY(stage_init());
-  const size_t per = STAGE_BYTES / width;
+  const size_t slice = stage_slice(width * cols, width);
+  DDC_TRY(stage_init(slice));
+  const size_t per = slice / width;
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
   for (size_t c0 = 0, i = 0; c0 < cols; ++i) {
@@ -272,13 +289,14 @@ static int copy_h2d(void* dst, size_t dpitch, const void* src, size_t spitch, si
 // device -> host (pageable); complete when it returns
 static int copy_d2h(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width,
                     size_t cols, hipStream_t st) {
-  if (width * cols < STAGE_MIN || width > STAGE_BYTES) {
+  if (width > STAGE_BYTES) {
     DDC_HIP(hipMemcpy2DAsync(dst, dpitch, src, spitch, width, cols, hipMemcpyDeviceToHost, st));
     DDC_HIP(hipStreamSynchronize(st));
     return DDC_OK;
   }
-  DDC_TRY(stage_init());
-  const size_t per = STAGE_BYTES / width;
+  const size_t slice = stage_slice(width * cols, width);
+  DDC_TRY(stage_init(slice));
+  const size_t per = slice / width;
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
   size_t pc0 = 0, pnc = 0;
@@ -698,8 +716,8 @@ static int bidiag_host(int m, int n, double* A, double* alpha, double* beta) {
   double* db = ws.take<double>(n);
   int* flag = ws.take<int>(64);
   DDC_HIP(hipMemsetAsync(Ap, 0, sizeof(double) * (size_t)lda_p * n, st));
-  DDC_HIP(hipMemcpy2DAsync(Ap, sizeof(double) * lda_p, A, sizeof(double) * m,
-                           sizeof(double) * m, n, hipMemcpyHostToDevice, st));
+  const size_t D = sizeof(double);
+  DDC_TRY(copy_h2d(Ap, D * lda_p, A, D * m, D * m, n, st));
   // extreme magnitudes: scaled by a power of two, alpha and beta scaled
   // back (the reflectors left in A are dimensionless); a matrix holding NaN
   // or Inf is bidiagonalized as it stands
@@ -709,12 +727,10 @@ static int bidiag_host(int m, int n, double* A, double* alpha, double* beta) {
   DDC_TRY(bidiag_run(m, n, Ap, lda_p, da, db, ws, st));
   DDC_TRY(unscale(std::min(m, n), da, aexp, st));
   DDC_TRY(unscale(nbeta, db, aexp, st));
-  DDC_HIP(hipMemcpy2DAsync(A, sizeof(double) * m, Ap, sizeof(double) * lda_p,
-                           sizeof(double) * m, n, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipMemcpyAsync(alpha, da, sizeof(double) * std::min(m, n), hipMemcpyDeviceToHost, st));
-  if (nbeta > 0)
-    DDC_HIP(hipMemcpyAsync(beta, db, sizeof(double) * nbeta, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(copy_d2h(A, D * m, Ap, D * lda_p, D * m, n, st));
+  const size_t wa = D * std::min(m, n), wb = D * nbeta;
+  DDC_TRY(copy_d2h(alpha, wa, da, wa, wa, 1, st));
+  if (nbeta > 0) DDC_TRY(copy_d2h(beta, wb, db, wb, wb, 1, st));
   return DDC_OK;
 }
 
@@ -766,10 +782,10 @@ static int bdsvd_host(int n, const double* alpha, const double* beta, double* si
       pb = sb.data();
     }
   }
-  DDC_HIP(hipMemcpyAsync(da, pa, sizeof(double) * n, hipMemcpyHostToDevice, st));
+  const size_t D = sizeof(double);
+  DDC_TRY(copy_h2d(da, D * n, pa, D * n, D * n, 1, st));
   DDC_HIP(hipMemsetAsync(db, 0, sizeof(double) * n, st));
-  if (n > 1)
-    DDC_HIP(hipMemcpyAsync(db, pb, sizeof(double) * (n - 1), hipMemcpyHostToDevice, st));
+  if (n > 1) DDC_TRY(copy_h2d(db, D * (n - 1), pb, D * (n - 1), D * (n - 1), 1, st));
   DDC_TRY(dc_run(n, da, db, ds, ws, st));
   if (vec) {
     double* Vt = ws.take<double>((size_t)ldb * n * 2);
@@ -778,14 +794,12 @@ static int bdsvd_host(int n, const double* alpha, const double* beta, double* si
     DDC_TRY(twisted_run(n, da, db, ds, Vt, Ut, ldb, ws, st));
     if (X) {
       DDC_TRY(transpose_f64(n, n, Vt, ldb, tmp, n, st));
-      DDC_HIP(hipMemcpyAsync(X, tmp, sizeof(double) * (size_t)n * n, hipMemcpyDeviceToHost, st));
-      DDC_HIP(hipStreamSynchronize(st));
+      DDC_TRY(copy_d2h(X, D * n, tmp, D * n, D * n, n, st));
       DDC_TRY(transpose_f64(n, n, Ut, ldb, tmp, n, st));
-      DDC_HIP(hipMemcpyAsync(Y, tmp, sizeof(double) * (size_t)n * n, hipMemcpyDeviceToHost, st));
+      DDC_TRY(copy_d2h(Y, D * n, tmp, D * n, D * n, n, st));
     }
   }
-  DDC_HIP(hipMemcpyAsync(sigma, ds, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(copy_d2h(sigma, D * n, ds, D * n, D * n, 1, st));
   if (scaled) {
     const double g1 = std::ldexp(1.0, aexp / 2), g2 = std::ldexp(1.0, aexp - aexp / 2);
     for (int i = 0; i < n; ++i) sigma[i] = sigma[i] * g1 * g2;
@@ -853,11 +867,10 @@ static int form_host(bool left, int m, int n, const double* A, double* Q) {
   double* Qd = ws.take<double>((size_t)k * k);
   if (!Qd) return DDC_E_NOMEM;
   DDC_HIP(hipMemsetAsync(Ap, 0, sizeof(double) * (size_t)lda_p * n, st));
-  DDC_HIP(hipMemcpy2DAsync(Ap, sizeof(double) * lda_p, A, sizeof(double) * m,
-                           sizeof(double) * m, n, hipMemcpyHostToDevice, st));
+  const size_t D = sizeof(double);
+  DDC_TRY(copy_h2d(Ap, D * lda_p, A, D * m, D * m, n, st));
   DDC_TRY(form_q_run(left, m, n, Ap, lda_p, Qd, k, ws, st));
-  DDC_HIP(hipMemcpyAsync(Q, Qd, sizeof(double) * (size_t)k * k, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(copy_d2h(Q, D * k, Qd, D * k, D * k, k, st));
   return DDC_OK;
 }
 
