@@ -101,8 +101,7 @@ int adjoint_run(int m, int n, const double* U, int ldu, const double* sigma,
   double* G = ws.take<double>((size_t)m * n);
   if (!G) return DDC_E_NOMEM;
   double smax = 0.0;
-  DDC_HIP(hipMemcpyAsync(&smax, sigma + (n - 1), sizeof(double), hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(host_read(&smax, sigma + (n - 1), sizeof(double), st));
 
   if (Ub) DDC_TRY(dgemm('T', 'N', n, n, m, 1.0, U, ldu, Ub, ldub, 0.0, P, n, st));
   if (Vb) DDC_TRY(dgemm('T', 'N', n, n, n, 1.0, V, ldv, Vb, ldvb, 0.0, Q, n, st));

@@ -1437,15 +1437,6 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
     }
   }
 
-  DDC_HIP(hipMemsetAsync(a.Y, 0, sizeof(double) * (size_t)d.ldy * NB * 2, st));
-  DDC_HIP(hipMemsetAsync(a.X, 0, sizeof(double) * (size_t)lda * NB, st));
-  DDC_HIP(hipMemsetAsync(beta, 0, sizeof(double) * n, st));
-
-  a.ncn = (int)ceil_div(m, 256);
-  a.nrn = 0;
-  hipLaunchKernelGGL(bd_init<TS>, dim3(a.ncn), dim3(256), 0, st, m, A, a.cvec, a.cnorm);
-  DDC_LAUNCHED();
-
   const int mn = std::min(m, n);
   // column steps whose two GEMVs are one pass (bd_fused_gemv): the plain
   // steps (not the last two columns or the wide last row) on at most
@@ -1456,6 +1447,22 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
   };
   // columns from this panel boundary on fit the register files (resident.hip)
   int res_k = fused_gemv_on() ? resident_first<TS>(m, n, NB) : -1;
+  // the panel operands' padding and the first column's norm: not needed where
+  // the steps run in registers from the first one on (four launches)
+  auto begin = [&](int k) {
+    DDC_HIP(hipMemsetAsync(a.Y, 0, sizeof(double) * (size_t)d.ldy * NB * 2, st));
+    DDC_HIP(hipMemsetAsync(a.X, 0, sizeof(double) * (size_t)lda * NB, st));
+    a.ncn = (int)ceil_div(m - k, 256);
+    a.nrn = 0;
+    hipLaunchKernelGGL(bd_init<TS>, dim3(a.ncn), dim3(256), 0, st, m - k, A + k + (int64_t)k * lda,
+                       a.cvec + k, a.cnorm);
+    DDC_LAUNCHED();
+    return DDC_OK;
+  };
+  if (res_k != 0) {
+    DDC_HIP(hipMemsetAsync(beta, 0, sizeof(double) * n, st));
+    DDC_TRY(begin(0));
+  }
   int fusedL = 0;  // tiles of left GEMV partials the trailing update left for step k, or 0
   int nfr_prev = 0;  // groups of the previous bd_right_fin (rows of its panel dots)
   for (int k = 0; k < mn; ++k) {
@@ -1472,10 +1479,7 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
       // from panel boundary `done` (resident_run is not tried again)
       res_k = -1;
       k = done - 1;
-      a.ncn = (int)ceil_div(m - done, 256);
-      hipLaunchKernelGGL(bd_init<TS>, dim3(a.ncn), dim3(256), 0, st, m - done,
-                         A + done + (int64_t)done * lda, a.cvec + done, a.cnorm);
-      DDC_LAUNCHED();
+      DDC_TRY(begin(done));
       continue;
     }
     if (m < n && k == m - 1) {

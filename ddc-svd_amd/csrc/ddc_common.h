@@ -145,6 +145,10 @@ int svd_device(int m, int n, const double* dA, int lda, double* dsigma, double* 
 
 // Singular values (ascending) of the n x (n+1) upper bidiagonal with diagonal
 // a[n] and super-diagonal b[n] by divide and conquer.
+// bytes (at most 4096) of device memory to the host through a pinned buffer,
+// after the work before them on st; waits for st
+int host_read(void* dst, const void* src, size_t bytes, hipStream_t st);
+
 void dc_plan(ArenaPlan& p, int n);
 int dc_run(int n, const double* a, const double* b, double* sigma, Arena& ws,
            hipStream_t st);

@@ -769,6 +769,11 @@ void resident_plan(ArenaPlan& p) {
 // block A[k0:m, k0:n] must be fully updated.  *done: the steps completed
 // (less than min(m, n) if a launch did not assemble; A is then fully updated
 // from *done, a multiple of align, on).
+__global__ __launch_bounds__(1024) void rs_clear(unsigned* sync, double* beta, int nb) {
+  for (int i = threadIdx.x; i < RS_SYNC; i += 1024) sync[i] = 0;
+  for (int i = threadIdx.x; i < nb; i += 1024) beta[i] = 0.0;
+}
+
 template <typename TS>
 int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int k0, int align,
                  Arena& ws, hipStream_t st, int* done) {
@@ -779,7 +784,9 @@ int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int 
   u64* ring = ws.take<u64>((size_t)mx);
   unsigned* sync = ws.take<unsigned>(RS_SYNC);
   if (!sync) return DDC_E_NOMEM;
-  DDC_HIP(hipMemsetAsync(sync, 0, sizeof(unsigned) * RS_SYNC, st));
+  // beta too where nothing before this call has cleared it
+  hipLaunchKernelGGL(rs_clear, dim3(1), dim3(1024), 0, st, sync, beta, k0 == 0 ? n : 0);
+  DDC_LAUNCHED();
   const int mn = std::min(m, n);
   int start[RS_LAUNCH];  // first step of each launch
   int nl = 0;
@@ -818,8 +825,7 @@ int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int 
     k = k1;
   }
   unsigned status = 0;
-  DDC_HIP(hipMemcpyAsync(&status, sync + RS_STATUS, sizeof(status), hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(host_read(&status, sync + RS_STATUS, sizeof(status), st));
   if (status == RS_FAILED) {
     report_error("an exchange of the bidiagonalization's work-groups gave up");
     return DDC_E_HIP;

@@ -1217,6 +1217,20 @@ __global__ void tw_identity(int n, double* Vt, double* Ut, int ldv, double* sigm
 
 static size_t tw_ck_size(int n) { return (size_t)((n + TW_CK - 1) / TW_CK) * 2 * n; }
 
+// out[0] = 1 if some value's square is within TW_GTOL (relative) of the one
+// before it, or below it.  If none is, the values increase, and so does any
+// subsequence of them (the lanes of one block), by more than TW_GTOL a step:
+// no two lanes form a group.
+__global__ __launch_bounds__(1024) void tw_close(int n, const double* sigma, int* out) {
+  int any = 0;
+  for (int j = 1 + threadIdx.x; j < n; j += 1024) {
+    const double s2 = sigma[j] * sigma[j], p2 = sigma[j - 1] * sigma[j - 1];
+    any |= s2 - p2 > TW_GTOL * s2 ? 0 : 1;
+  }
+  any = __syncthreads_or(any);
+  if (threadIdx.x == 0) out[0] = any ? 1 : 0;
+}
+
 void twisted_plan(ArenaPlan& p, int n) {
   p.add<double>(6 * (size_t)n);        // qd
   p.add<double>(2 * tw_ck_size(n));    // checkpoints
@@ -1254,8 +1268,7 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
   hipLaunchKernelGGL(tw_scale, dim3(1), dim3(1024), 0, st, n, a, b, sigma, scr);
   DDC_LAUNCHED();
   double hsc[3] = {0.0, 0.0, 0.0};
-  DDC_HIP(hipMemcpyAsync(hsc, scr, sizeof(hsc), hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  DDC_TRY(host_read(hsc, scr, sizeof(hsc), st));
   if (hsc[2] != 0.0 || !(hsc[0] < INFINITY)) {
     report_error("singular values of the bidiagonal are not finite");
     return DDC_E_NUMERIC;
@@ -1318,15 +1331,24 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
 
   // groups: lanes of one block whose refined values are within TW_GTOL
   // (relative, in sigma^2) of the block's previous lane
-  std::vector<int> hblk(n), hbe(n);
-  std::vector<double> hs(n);
-  DDC_HIP(hipMemcpyAsync(hblk.data(), blk, sizeof(int) * n, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipMemcpyAsync(hbe.data(), be, sizeof(int) * n, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipMemcpyAsync(hs.data(), sigma, sizeof(double) * n, hipMemcpyDeviceToHost, st));
-  DDC_HIP(hipStreamSynchronize(st));
+  // -- only where some pair of neighbouring values is that close, which
+  // tw_close tells in one word: else all n are further apart, of whatever block
+  hipLaunchKernelGGL(tw_close, dim3(1), dim3(1024), 0, st, n, sigma, cnt);
+  DDC_LAUNCHED();
+  int any = 0;
+  DDC_TRY(host_read(&any, cnt, sizeof(int), st));
+  const int nh = any ? n : 0;  // lanes to group
+  std::vector<int> hblk(nh), hbe(nh);
+  std::vector<double> hs(nh);
+  if (any) {
+    DDC_HIP(hipMemcpyAsync(hblk.data(), blk, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+    DDC_HIP(hipMemcpyAsync(hbe.data(), be, sizeof(int) * n, hipMemcpyDeviceToHost, st));
+    DDC_HIP(hipMemcpyAsync(hs.data(), sigma, sizeof(double) * n, hipMemcpyDeviceToHost, st));
+    DDC_HIP(hipStreamSynchronize(st));
+  }
   // per block: its last lane, the first lane and size of its open group;
   // members of a group are chained through nxt
-  std::vector<int> last(n, -1), gst(n, -1), gsz(n, 0), nxt(n, -1);
+  std::vector<int> last(nh, -1), gst(nh, -1), gsz(nh, 0), nxt(nh, -1);
   // A group is cut into windows of TW_KMAX members (the last may hold
   // one); window w of a group runs in launch w, after the group's earlier
   // windows, against whose final vectors it is orthogonalised.
@@ -1345,7 +1367,7 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
       lvl.push_back((int)(w / TW_KMAX));
     }
   };
-  for (int j = 0; j < n; ++j) {
+  for (int j = 0; j < nh; ++j) {
     const int kb = std::min(std::max(hblk[j], 0), n - 1);
     const int p = last[kb];
     const double s2 = hs[j] * hs[j];
@@ -1359,7 +1381,7 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
     }
     last[kb] = j;
   }
-  for (int kb = 0; kb < n; ++kb)
+  for (int kb = 0; kb < nh; ++kb)
     if (last[kb] >= 0) close(kb);
   if (!tab.empty()) {
     // windows in launch order: every group's first window, then the second ...
