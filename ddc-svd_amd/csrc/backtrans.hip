@@ -5,11 +5,12 @@
 // time (BLAS1).  Here the reflectors stored in A are grouped into blocks of
 // NBB and applied in compact WY form,
 //     H_k0 ... H_{k0+NBB-1} = I - W T W^T,   T upper triangular,
-// for the unit-norm convention H = I - 2 w w^T (tau = 2).  T is never formed:
-// its inverse is T^{-1} = I/2 + strict_upper(W^T W) (the identity behind
+// for the unit-norm convention H = I - 2 w w^T (tau = 2).  The inverse of T is
+// T^{-1} = I/2 + strict_upper(W^T W) (the identity behind
 // the recursive T-factor of LAPACK dlarft), so a block costs
-//     G = W^T W,  Z = W^T C,  Z = T Z (triangular solve with T^{-1}),
-//     C -= W Z
+//     G = W^T W,  Z = W^T C,  Z = T Z,  C -= W Z
+// (in FP64 T is formed from G by bt_tdiag and bt_tmerge and applied as a
+// product, elsewhere by a triangular solve with T^{-1})
 // with the block's reflectors first packed into a dense zero-padded W; the
 // three products are library GEMMs (rocBLAS, FP64 MFMA).
 // Left reflectors are the columns A[k:m, k]; right reflectors are the rows
@@ -96,14 +97,152 @@ __global__ void bt_pack(int rows, int nb, const T* S, int lda, T* Wd, int ldw) {
 // T^{-1} = I/2 + strict_upper(G) (nb x nb, ld nb) for the block
 // H_0 ... H_{nb-1} = I - W T W^T of unit-norm reflectors (tau = 2).
 template <typename T>
-__global__ void bt_tinv(int nb, T* G, T* Ti) {
+__global__ void bt_tinv(int nb, const T* G, T* Ti) {
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= nb * nb) return;
   const int i = e % nb, j = e / nb;
   Ti[e] = i < j ? G[e] : (i == j ? T(0.5) : T(0));
-  // G's strict lower part to zero: G then receives T (upper triangle only)
-  // and is used as a full matrix
-  if (i > j) G[e] = T(0);
+}
+
+// T (nb x nb, ld nb, zeros below the diagonal) from G = W^T W in two kernels:
+// the 64 x 64 diagonal blocks of I/2 + strict_upper(G) are inverted in LDS
+// (bt_tdiag), then ever larger pairs of inverted blocks are joined (bt_tmerge,
+// one launch per doubling):
+//     [A B; 0 C]^{-1} = [A^{-1}, -A^{-1} B C^{-1}; 0, C^{-1}].
+// A block's chain of dependent launches is what it costs, not its arithmetic
+// (a 512 x 512 T is 0.1 GFLOP): one to four launches instead of the 8 to 11 of
+// the library's triangular inverse took the back-transformation from 0.25 to
+// 0.13 ms at 96 x 64, 0.37 to 0.22 at 512 x 256 and 1.17 to 0.98 at
+// 1531 x 1187.
+constexpr int TB = 64;
+
+__global__ __launch_bounds__(256) void bt_tdiag(int nb, const double* G, double* T) {
+  const int tid = threadIdx.x;
+  const int i0 = blockIdx.x * TB, j0 = blockIdx.y * TB;
+  if (i0 < j0) return;
+  if (i0 > j0) {
+    for (int e = tid; e < TB * TB; e += 256) {
+      const int i = i0 + e % TB, j = j0 + e / TB;
+      if (i < nb && j < nb) T[i + (int64_t)j * nb] = 0.0;
+    }
+    return;
+  }
+  __shared__ double U[TB][TB + 1];  // U[j][i]: entry (i, j), inverted in place
+  __shared__ double P[32 * 32];
+  for (int e = tid; e < TB * TB; e += 256) {
+    const int i = e % TB, j = e / TB;
+    U[j][i] = i < j ? (j0 + j < nb ? G[i0 + i + (int64_t)(j0 + j) * nb] : 0.0)
+                    : (i == j ? 0.5 : 0.0);
+  }
+  __syncthreads();
+  // the four 16 x 16 diagonal blocks, a lane per column: back substitution
+  if (tid < 64) {
+    const int base = tid & 48, j = tid & 15;
+    double x[16];
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+      double sum = 0.0;
+#pragma unroll
+      for (int k = i + 1; k < 16; ++k) sum += U[base + k][base + i] * x[k];
+      x[i] = i == j ? 2.0 : (i < j ? -2.0 * sum : 0.0);
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) U[base + j][base + i] = x[i];
+  }
+  __syncthreads();
+  for (int s = 16; s < TB; s *= 2) {
+    const int tot = TB / 2 * s;  // entries of the TB / (2 s) pairs' B blocks
+    for (int e = tid; e < tot; e += 256) {
+      const int i = e % s, j = e / s % s, r0 = e / (s * s) * 2 * s;
+      double sum = 0.0;
+      for (int k = 0; k <= j; ++k) sum += U[r0 + s + k][r0 + i] * U[r0 + s + j][r0 + s + k];
+      P[e] = sum;
+    }
+    __syncthreads();
+    for (int e = tid; e < tot; e += 256) {
+      const int i = e % s, j = e / s % s, q = e / (s * s), r0 = q * 2 * s;
+      double sum = 0.0;
+      for (int k = i; k < s; ++k) sum += U[r0 + k][r0 + i] * P[q * s * s + j * s + k];
+      U[r0 + s + j][r0 + i] = -sum;
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < TB * TB; e += 256) {
+    const int i = e % TB, j = e / TB;
+    if (i0 + i < nb && j0 + j < nb) T[i0 + i + (int64_t)(j0 + j) * nb] = U[j][i];
+  }
+}
+
+// Joins the inverted s x s blocks A (rows r0 = 2 s blockIdx.y) and C (rows
+// r0 + s): a group takes 16 columns of the s x s block between them, first
+// X = B C^{-1}, kept in LDS, then -A^{-1} X, in 16 x 16 FP64 matrix-core
+// blocks over 8 waves (operand layouts: gemm.hip).  s a multiple of 16 up to
+// 256; columns from nb on are zeros.
+__global__ __launch_bounds__(512) void bt_tmerge(int nb, int s, const double* G, double* T) {
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  __shared__ double X[256 * 17];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = 2 * s * blockIdx.y, c0 = blockIdx.x * 16;
+  const int rc = r0 + s, col = rc + c0;  // C's first row, this group's first column
+  if (col >= nb) return;
+  const int kc = c0 + 16;  // rows of C^{-1} above this panel's diagonal
+  for (int e = tid; e < kc * 16; e += 512) {
+    const int k = e % kc, c = e / kc;
+    X[k * 17 + c] = rc + k < nb && col + c < nb ? T[rc + k + (int64_t)(col + c) * nb] : 0.0;
+  }
+  __syncthreads();
+  d4 acc[2] = {d4{0, 0, 0, 0}, d4{0, 0, 0, 0}};
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int t = wave + 8 * q;
+    if (16 * t >= s) break;
+    const double* g = G + r0 + 16 * t + lr + (int64_t)rc * nb;
+#pragma unroll 4
+    for (int k = 0; k < kc; k += 4) {
+      const double av = rc + k + lq < nb ? g[(int64_t)(k + lq) * nb] : 0.0;
+      acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, X[(k + lq) * 17 + lr], acc[q], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int t = wave + 8 * q;
+    if (16 * t >= s) break;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) X[(16 * t + lq + 4 * r) * 17 + lr] = acc[q][r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int t = wave + 8 * q;
+    if (16 * t >= s) break;
+    const double* a = T + r0 + 16 * t + lr + (int64_t)r0 * nb;
+    d4 sum = {0, 0, 0, 0};
+#pragma unroll 4
+    for (int k = 16 * t; k < s; k += 4)
+      sum = __builtin_amdgcn_mfma_f64_16x16x4f64(a[(int64_t)(k + lq) * nb],
+                                                 X[(k + lq) * 17 + lr], sum, 0, 0, 0);
+    if (col + lr < nb) {
+      double* o = T + r0 + 16 * t + (int64_t)(col + lr) * nb;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[lq + 4 * r] = -sum[r];
+    }
+  }
+}
+
+static int form_t(int nb, const double* G, double* T, hipStream_t st) {
+  static_assert(NBB <= 512, "bt_tmerge joins blocks of up to 256");
+  const unsigned nt = (unsigned)ceil_div(nb, TB);
+  hipLaunchKernelGGL(bt_tdiag, dim3(nt, nt), dim3(256), 0, st, nb, G, T);
+  DDC_LAUNCHED();
+  for (int s = TB; s < nb; s *= 2) {
+    hipLaunchKernelGGL(bt_tmerge, dim3(s / 16, (unsigned)ceil_div(nb, 2 * s)), dim3(512), 0, st,
+                       nb, s, G, T);
+    DDC_LAUNCHED();
+  }
+  return DDC_OK;
 }
 
 // Library GEMM / triangular solve in the precision of the block.
@@ -146,7 +285,7 @@ static int side_stream(SideStream** out) {
 }
 
 void backtrans_plan(ArenaPlan& p, int m, int n) {
-  p.add<double>((size_t)NBB * NBB * 2);  // G (then T), T^{-1}
+  p.add<double>((size_t)NBB * NBB * 2);  // G, T
   p.add<double>((size_t)NBB * n);        // Z
   p.add<double>((size_t)m * NBB);        // packed reflectors
   p.add<double>((size_t)NBB * n);        // T Z
@@ -158,11 +297,10 @@ void backtrans_plan(ArenaPlan& p, int m, int n) {
 }
 
 // Apply H_k0 ... H_k1-1 (blocks, last block first) to the rows of C:
-// Z = W^T C, Z = T Z, C -= W Z.  With Z2 (FP64): T is formed once per block
-// from T^{-1} (triangular inverse of the nb x nb matrix) and applied as a
-// GEMM into Z2 (nb x ncol); else by a triangular solve with T^{-1} in place
-// (the solve's blocked small products took about a third of the
-// back-transformation at 8192^2).
+// Z = W^T C, Z = T Z, C -= W Z.  With Z2 (FP64 only): T is formed once per
+// block into Ti and applied as a GEMM into Z2 (nb x ncol); else by a triangular
+// solve with T^{-1} in place (the solve's blocked small products took about a
+// third of the back-transformation at 8192^2).
 // left: w_k = A[k:m, k];  right: w_k = A[k, k+1:n] acting on rows k+1..n-1.
 template <typename T>
 static int apply_blocks(bool left, int m, int n, const T* A, int lda, int nref, T* C, int ldc,
@@ -183,20 +321,19 @@ static int apply_blocks(bool left, int m, int n, const T* A, int lda, int nref, 
                          A + k0 + (int64_t)(k0 + 1) * lda, lda, Wd, rows);
     DDC_LAUNCHED();
     DDC_TRY(gemm_t('T', 'N', nb, nb, rows, T(1), Wd, rows, Wd, rows, T(0), G, nb, st));
-    hipLaunchKernelGGL(bt_tinv<T>, dim3((unsigned)ceil_div(nb * nb, 256)), dim3(256), 0, st, nb,
-                       G, Ti);
-    DDC_LAUNCHED();
     DDC_TRY(gemm_t('T', 'N', nb, ncol, rows, T(1), Wd, rows, Csub, ldc, T(0), Z, nb, st));
-    T* Zt = Z;
-    if constexpr (sizeof(T) == 8) {
-      if (Z2) {
-        // T = (T^{-1})^{-1} into G (no longer needed), then Z2 = T Z
-        DDC_TRY(dtrtri_upper(nb, Ti, nb, G, nb, st));
-        DDC_TRY(gemm_t('N', 'N', nb, ncol, nb, T(1), G, nb, Z, nb, T(0), Z2, nb, st));
-        Zt = Z2;
+    T* Zt = Z2 ? Z2 : Z;
+    if (Z2) {
+      if constexpr (sizeof(T) == 8) {
+        DDC_TRY(form_t(nb, G, Ti, st));
+        DDC_TRY(gemm_t('N', 'N', nb, ncol, nb, T(1), Ti, nb, Z, nb, T(0), Z2, nb, st));
       }
+    } else {
+      hipLaunchKernelGGL(bt_tinv<T>, dim3((unsigned)ceil_div(nb * nb, 256)), dim3(256), 0, st, nb,
+                         G, Ti);
+      DDC_LAUNCHED();
+      DDC_TRY(trsm_t(nb, ncol, Ti, nb, Z, nb, st));
     }
-    if (Zt == Z) DDC_TRY(trsm_t(nb, ncol, Ti, nb, Z, nb, st));
     DDC_TRY(gemm_t('N', 'N', rows, ncol, nb, T(-1), Wd, rows, Zt, nb, T(1), Csub, ldc, st));
   }
   return DDC_OK;
