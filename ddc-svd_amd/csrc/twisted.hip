@@ -65,6 +65,7 @@ constexpr double TW_GTOL = 1e-6;   // relative gap (in sigma^2) that forms a gro
 constexpr int TW_KMAX = 64;        // members per Rayleigh-Ritz window
 constexpr double TW_TIGHT = 1024.0;  // members closer than this (eps, relative) share a shift
 constexpr int TW_RRIT = 3;          // inverse-iteration steps per Rayleigh-Ritz member
+constexpr unsigned TW_CUS = 256;    // CUs of the GPU
 constexpr int TW_CK = 64;          // checkpoint interval = LDS chunk
 constexpr int TW_MAXBIS = 200;     // bisection steps per lane at most
 constexpr double TW_CONV = 32.0;   // Rayleigh correction accepted below TW_CONV eps lam
@@ -375,23 +376,30 @@ struct TwArgs {
   int* blk;              // out: block start of the lane's vector (rep 0)
 };
 
-// Two waves per group of 64 singular values, all lanes on the same
-// representation; lane = one singular value, and lane l of both waves works
+// 2 H waves per group of 64 singular values, all lanes on the same
+// representation; lane = one singular value, and lane l of all waves works
 // on the same value (their per-value state is kept identical).  The lanes
 // walk the index range in lockstep, chunk by chunk; the chunk's qd entries
 // are staged in LDS, and the recurrences that a pass needs in the opposite
 // direction are recomputed for the chunk from checkpoints (every TW_CK
 // steps) into a per-wave LDS buffer.  Nothing of size n per lane is stored
-// except the vector itself.  The two waves run the independent recurrences
-// of each pass side by side, on different SIMDs:
+// except the vector itself.  Even waves (side 0) and odd ones (side 1) run the
+// independent recurrences of each pass side by side, on different SIMDs:
 //   pass 1   wave 0: stationary transform, ascending (checkpoints of s,
 //            Sturm count at lam); wave 1: progressive transform,
 //            descending (checkpoints of p)
-//   pass 2   per chunk, wave 0 recomputes s and wave 1 recomputes p; gamma
+//   pass 2   per chunk, side 0 recomputes s and side 1 recomputes p; gamma
 //            and its argmin over the chunk's two halves, among the indices
 //            of the lane's twist range
-//   pass 3   wave 0: z downward from the twist (recomputed p); wave 1: z
+//   pass 3   side 0: z downward from the twist (recomputed p); side 1: z
 //            upward (recomputed s)
+// What bounds the kernel is the chain of divisions of one lane, n long in
+// each pass.  Between checkpoints passes 2 and 3 need no such chain: with
+// H = 2 each pair of waves takes every other chunk, in pass 3 up to the
+// quotients; only the product z = q z, without a division, then runs through
+// the chunks in order (in waves 0 and 1).  Every value is formed as with
+// H = 1, bit for bit.  The vectors stage went from 0.26 to 0.21 ms at
+// 512 x 256, 1.01 to 0.81 at 1531 x 1187 and 14.1 to 10.1 at 8192 x 8192.
 //
 // Recurrences (L D L^T - lam I, d = a^2, ld = a b, lld = b^2; lld_i = 0
 // restarts them, B being block diagonal there):
@@ -403,13 +411,15 @@ struct TwArgs {
 //   vector      z_r = 1, z_{i+1} = -(ld_i / D-_{i+1}) z_i  (i >= r),
 //               z_i = -(ld_i / D+_i) z_{i+1}  (i < r)
 //   correction  lam += gamma_r / |z|^2   (Rayleigh quotient)
-__global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
+template <int H>
+__global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
+  constexpr int NW = 2 * H;
   // staged qd of the chunk each wave works on: [wave][d, ld, lld][e]
-  __shared__ double qs[2][3][TW_CK];
-  __shared__ double buf[2][TW_CK][64];  // per-wave recomputed s or p, [e][lane]
+  __shared__ double qs[NW][3][TW_CK];
+  __shared__ double buf[NW][TW_CK][64];  // per-wave s, p, quotients or z, [e][lane]
   // exchange between the waves, [wave][lane]
-  __shared__ double xg[2][64], xn[2][64];
-  __shared__ int xr[2][64], xc[64];
+  __shared__ double xg[NW][64], xn[2][64];
+  __shared__ int xr[NW][64], xc[64];
   const int n = a.n;
   const int nbr = (n + 63) / 64;
   const int rep = ((int)blockIdx.x >= nbr) ? 1 : 0;
@@ -417,6 +427,7 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
   // so the full-chunk loops below are straight-line code
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int side = wave & 1, half = wave >> 1;
   const int idx = ((int)blockIdx.x - rep * nbr) * 64 + lane;
   const bool live = idx < n;
   const int li = live ? idx : 0;
@@ -429,7 +440,7 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
   const int64_t ldv = a.ldv;
   auto oidx = [&](int j) -> int64_t { return (int64_t)(rep ? (n - 1 - j) : j) * ldv; };
   const int nck = (n + TW_CK - 1) / TW_CK;
-  // both waves stage one chunk each (cw: this wave's chunk)
+  // every wave stages one chunk (cw: this wave's chunk)
   auto stage = [&](int cw) {
     __syncthreads();
     const int c0 = cw * TW_CK, len = min(TW_CK, n - c0);
@@ -469,7 +480,7 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
   int rfin = g1 - 1;
   bool active = live;
   for (int it = 0; it < 10; ++it) {
-    if (__ballot(active) == 0) break;  // the same in both waves
+    if (__ballot(active) == 0) break;  // the same in all waves
     // pass 1: stationary (wave 0, ascending) and progressive (wave 1,
     // descending) transforms with checkpoints
     int cnt = 0;
@@ -477,7 +488,7 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
       double s = -lam;           // wave 0
       double p = dn1 - lam;      // wave 1
       for (int c = 0; c < nck; ++c) {
-        const int cw = wave == 0 ? c : nck - 1 - c;
+        const int cw = side == 0 ? c : nck - 1 - c;
         stage(cw);
         const int c0 = cw * TW_CK, len = min(TW_CK, n - c0);
         if (wave == 0) {
@@ -493,7 +504,7 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
           } else {
             for (int e = 0; e < len; ++e) step(e);
           }
-        } else {
+        } else if (wave == 1) {
           auto step = [&](int e) {
             const double dm = guard(qd_lld[e] + p, pivmin);
             p = prog_prev(p, qd_d[e], dm, qd_lld[e], lam);
@@ -513,10 +524,13 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
     // pass 2: gamma_i = s_i + p_i + lam over each chunk, both recomputed
     int r = -1;  // no finite candidate yet
     double gbest = INFINITY;
-    for (int c = 0; c < nck; ++c) {
-      stage(c);
-      const int c0 = c * TW_CK, len = min(TW_CK, n - c0);
-      if (wave == 0) {
+    for (int cb = 0; cb < nck; cb += H) {
+      const int c = cb + half;
+      stage(min(c, nck - 1));
+      // a chunk past the last one: no entries
+      const int c0 = c * TW_CK, len = max(0, min(TW_CK, n - c0));
+      if (len == 0) {
+      } else if (side == 0) {
         double ss = Sck[(int64_t)c * T];
         auto step = [&](int e) {
           bw[e][lane] = ss;
@@ -551,13 +565,13 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
         }
       }
       __syncthreads();
-      // wave 0 takes e < 32 of the chunk, wave 1 e >= 32
+      // side 0 takes e < 32 of the chunk, side 1 e >= 32
 #pragma unroll 4
       for (int q = 0; q < TW_CK / 2; ++q) {
-        const int e = wave * (TW_CK / 2) + q;
+        const int e = side * (TW_CK / 2) + q;
         const int i = c0 + e;
         if (e < len && i >= g0 && i < g1) {
-          const double g = buf[0][e][lane] + buf[1][e][lane] + lam;
+          const double g = buf[2 * half][e][lane] + buf[2 * half + 1][e][lane] + lam;
           if (fabs(g) < fabs(gbest) || (fabs(g) == fabs(gbest) && fabs(g) < INFINITY)) {
             gbest = g;
             r = i;
@@ -572,95 +586,111 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
       xr[wave][lane] = r;
       if (wave == 0) xc[lane] = cnt;
       __syncthreads();
-      const double g0v = xg[0][lane], g1v = xg[1][lane];
-      const int rr0 = xr[0][lane], rr1 = xr[1][lane];
       cnt = xc[lane];
-      const bool take1 = rr1 >= 0 &&
-                         (rr0 < 0 || fabs(g1v) < fabs(g0v) || (fabs(g1v) == fabs(g0v) && rr1 > rr0));
-      if (take1) {
-        gbest = g1v;
-        r = rr1;
-      } else if (rr0 >= 0) {
-        gbest = g0v;
-        r = rr0;
-      } else {
-        gbest = INFINITY;
-        r = g1 - 1;
+      r = -1;
+      gbest = INFINITY;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const double gw = xg[w][lane];
+        const int rw = xr[w][lane];
+        if (rw >= 0 && (r < 0 || fabs(gw) < fabs(gbest) || (fabs(gw) == fabs(gbest) && rw > r))) {
+          gbest = gw;
+          r = rw;
+        }
       }
+      if (r < 0) r = g1 - 1;
     }
-    // pass 3: wave 0 z downward from r (needs p_{i+1}), wave 1 upward (s_i)
-    double nzp = wave == 0 ? 1.0 : 0.0;
+    // pass 3: side 0 z downward from r (needs p_{i+1}), side 1 upward (s_i):
+    // the chunk's quotients, the products through them, the stores
+    double nzp = side == 0 ? 1.0 : 0.0;
     if (active && wave == 0) out[oidx(r)] = 1.0;
     {
       double z = 1.0;
-      for (int c = 0; c < nck; ++c) {
-        const int cw = wave == 0 ? c : nck - 1 - c;
+      // chunk h of a round: first index and the entries it has a step for
+      auto chunk = [&](int kth) { return side == 0 ? kth : nck - 1 - kth; };
+      auto steps = [&](int kth) {
+        if (kth >= nck) return 0;
+        const int cw = chunk(kth);
+        const int len = min(TW_CK, n - cw * TW_CK);
+        return side == 0 && cw + 1 == nck ? len - 1 : len;
+      };
+      for (int k0 = 0; k0 < nck; k0 += H) {
+        const int kth = k0 + half, ns = steps(kth);
+        const int cw = chunk(min(kth, nck - 1)), c0 = cw * TW_CK;
         stage(cw);
-        const int c0 = cw * TW_CK, len = min(TW_CK, n - c0);
-        if (wave == 0) {
-          double pp;
-          int etop;
-          if (cw + 1 < nck) {
-            pp = Pck[(int64_t)(cw + 1) * T];  // p_{c0+len}
-            etop = len - 1;
-          } else {
-            pp = dn1 - lam;  // p_{n-1}
-            etop = len - 2;
-          }
-          auto pstep = [&](int e) {
-            bw[e][lane] = pp;  // p_{c0+e+1}
+        if (kth >= nck) {
+        } else if (side == 0) {
+          double pp = cw + 1 < nck ? Pck[(int64_t)(cw + 1) * T]  // p_{c0+len}
+                                   : dn1 - lam;                  // p_{n-1}
+          auto step = [&](int e) {  // pp = p_{c0+e+1}
             const double dm = guard(qd_lld[e] + pp, pivmin);
+            bw[e][lane] = -(qd_ld[e] / dm);
             pp = prog_prev(pp, qd_d[e], dm, qd_lld[e], lam);
           };
-          if (etop == TW_CK - 1) {
+          if (ns == TW_CK) {
 #pragma unroll 8
-            for (int e = TW_CK - 1; e >= 0; --e) pstep(e);
+            for (int e = TW_CK - 1; e >= 0; --e) step(e);
           } else {
-            for (int e = etop; e >= 0; --e) pstep(e);
-          }
-          // z in straight-line code (the quotient formed on every step and
-          // kept where the step applies), staged in bw and stored after
-#pragma unroll 8
-          for (int e = 0; e < TW_CK; ++e) {
-            const bool go = e <= etop && active && c0 + e >= r;
-            const double zn = keep(-(qd_ld[e] / guard(qd_lld[e] + bw[e][lane], pivmin)) * z);
-            z = go ? zn : z;
-            nzp += go ? zn * zn : 0.0;
-            bw[e][lane] = zn;
-          }
-          for (int e = 0; e < TW_CK; ++e) {
-            const int i = c0 + e;
-            if (e <= etop && active && i >= r) out[oidx(i + 1)] = bw[e][lane];
+            for (int e = ns - 1; e >= 0; --e) step(e);
           }
         } else {
           double ss = Sck[(int64_t)cw * T];
-          auto sstep = [&](int e) {
-            bw[e][lane] = ss;
+          auto step = [&](int e) {
             const double dp = guard(qd_d[e] + ss, pivmin);
+            bw[e][lane] = -(qd_ld[e] / dp);
             ss = stat_next(ss, dp, qd_lld[e], lam);
           };
-          if (len == TW_CK) {
+          if (ns == TW_CK) {
 #pragma unroll 8
-            for (int e = 0; e < TW_CK; ++e) sstep(e);
+            for (int e = 0; e < TW_CK; ++e) step(e);
           } else {
-            for (int e = 0; e < len; ++e) sstep(e);
+            for (int e = 0; e < ns; ++e) step(e);
           }
+        }
+        if (H > 1) __syncthreads();
+        if (half == 0) {
+          // z in straight-line code: the product formed on every step and
+          // kept where the step applies
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            const int nh = steps(k0 + h), ch = chunk(k0 + h) * TW_CK;
+            double (*bh)[64] = buf[2 * h + side];
+            if (side == 0) {
 #pragma unroll 8
-          for (int e = TW_CK - 1; e >= 0; --e) {
-            const bool go = e < len && active && c0 + e < r;
-            const double zn = keep(-(qd_ld[e] / guard(qd_d[e] + bw[e][lane], pivmin)) * z);
-            z = go ? zn : z;
-            nzp += go ? zn * zn : 0.0;
-            bw[e][lane] = zn;
+              for (int e = 0; e < TW_CK; ++e) {
+                const bool go = e < nh && active && ch + e >= r;
+                const double zn = keep(bh[e][lane] * z);
+                z = go ? zn : z;
+                nzp += go ? zn * zn : 0.0;
+                bh[e][lane] = zn;
+              }
+            } else {
+#pragma unroll 8
+              for (int e = TW_CK - 1; e >= 0; --e) {
+                const bool go = e < nh && active && ch + e < r;
+                const double zn = keep(bh[e][lane] * z);
+                z = go ? zn : z;
+                nzp += go ? zn * zn : 0.0;
+                bh[e][lane] = zn;
+              }
+            }
           }
-          for (int e = TW_CK - 1; e >= 0; --e) {
+        }
+        if (H > 1) __syncthreads();
+        if (side == 0) {
+          for (int e = 0; e < ns; ++e) {
             const int i = c0 + e;
-            if (e < len && active && i < r) out[oidx(i)] = bw[e][lane];
+            if (active && i >= r) out[oidx(i + 1)] = bw[e][lane];
+          }
+        } else {
+          for (int e = ns - 1; e >= 0; --e) {
+            const int i = c0 + e;
+            if (active && i < r) out[oidx(i)] = bw[e][lane];
           }
         }
       }
     }
-    xn[wave][lane] = nzp;
+    if (half == 0) xn[side][lane] = nzp;
     __syncthreads();
     // converged lanes keep the norm of their final vector
     if (active) {
@@ -691,11 +721,11 @@ __global__ __launch_bounds__(128) void tw_solve(TwArgs a) {
     if (!(nl > lo && nl < hi)) nl = 0.5 * (lo + hi);
     lam = nl;
   }
-  __syncthreads();  // both waves' vector entries are written
+  __syncthreads();  // all waves' vector entries are written
   if (!live) return;
   const double inv = 1.0 / sqrt(nz2);
-  const int jh = (n + 1) / 2;
-  const int ja = wave == 0 ? 0 : jh, jb = wave == 0 ? jh : n;
+  const int jh = (n + NW - 1) / NW;
+  const int ja = min(n, wave * jh), jb = min(n, ja + jh);
   for (int j0 = ja; j0 < jb; j0 += 8) {
     double v[8];
 #pragma unroll
@@ -1326,7 +1356,15 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
   t.flags = flags;
   t.bs = bs;
   t.blk = blk;
-  hipLaunchKernelGGL(tw_solve, dim3(2 * (unsigned)ceil_div(n, 64)), dim3(128), 0, st, t);
+  // Four waves (141 KiB of LDS, one group per CU) as long as the groups find a
+  // CU each; beyond, two waves, of which a CU holds two groups (vectors stage,
+  // four against two waves: n = 8192, 256 groups, 10.1 and 14.1 ms; n = 12288,
+  // 384 groups, 74 and 20.9 ms).
+  const unsigned ng = 2 * (unsigned)ceil_div(n, 64);
+  if (ng <= TW_CUS)
+    hipLaunchKernelGGL(tw_solve<2>, dim3(ng), dim3(256), 0, st, t);
+  else
+    hipLaunchKernelGGL(tw_solve<1>, dim3(ng), dim3(128), 0, st, t);
   DDC_LAUNCHED();
 
   // groups: lanes of one block whose refined values are within TW_GTOL
