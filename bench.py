@@ -259,7 +259,8 @@ def plain_form(m: int, n: int, seed: int = 2, steps: int = 3) -> dict:
     return {"config": f"plain FP64 svd_gpu {m}x{n}, N(0,1) entries, seed {seed}, "
                       f"device-resident input", "ms": 1e3 * sec, "svd_per_s": 1.0 / sec,
             "steps": steps, "stages_ms": {k: stage[k] for k in ddcsvd.TIMING_KEYS[:6]},
-            "bidiag_GBs": sum(gemv_bytes(max(m, n), min(m, n)).values())
+            # as if every step read its trailing block (those in registers do not)
+            "bidiag_GBs": sum(gemv_bytes(max(m, n), mn, mn).values())
                           / (stage["bidiag"] / 1e3) / 1e9,
             "residual": res, "orth_u": ou, "orth_v": ov}
 

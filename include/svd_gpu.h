@@ -204,7 +204,7 @@ int svd_gpu_batched_run(svd_gpu_batch *plan, const void *dA, void *dsigma,
  * batches); writes the outputs.  Synchronous. */
 int svd_gpu_batched_tune(svd_gpu_batch *plan, const void *dA, void *dsigma,
                          void *dU, void *dV, void *stream);
-/* Chosen configuration: kernel variant, resident 4-wave workgroups per CU,
+/* Chosen configuration: kernel variant, resident workgroups per CU,
  * the smallest min(m, n) that a whole workgroup factors together, and the
  * column-block widths for matrices of up to 128 / up to 256 rows.  Returns
  * the number of variants (variant = -1 before tuning). */
@@ -222,8 +222,8 @@ void svd_gpu_batched_destroy(svd_gpu_batch *plan);
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the batched SVD without a plan, with the same packed
  * buffer layout as svd_gpu_batched_offsets and the same kernel as
- * svd_gpu_batched_run, at a fixed launch configuration (variant 1, two
- * workgroups per CU, cooperation from min(m, n) = 32).  Its descriptors,
+ * svd_gpu_batched_run, at a fixed launch configuration (variant 1, one
+ * workgroup per CU, cooperation from min(m, n) = 32).  Its descriptors,
  * queue head and working copies live in a 32 MiB device array that each GPU
  * holds from the library's first kernel launch until the process ends; a
  * batch needing more (about sum of max(m,n) min(m,n) + min(m,n)^2 elements,
