@@ -197,8 +197,10 @@ static size_t stage_slice(size_t bytes, size_t width) {
   return std::min(STAGE_BYTES, std::max({STAGE_SLICE, width, bytes / 3}));
 }
 
-// two buffers of at least slice bytes
-static int stage_init(size_t slice) {
+// two buffers of at least slice bytes; *ok = false if the memory cannot be
+// pinned (the copy then goes directly)
+static int stage_init(size_t slice, bool* ok) {
+  *ok = true;
   if (g_ctx.stage_cap >= slice) return DDC_OK;
   size_t cap = STAGE_SLICE;
   while (cap < slice) cap *= 2;
@@ -208,7 +210,13 @@ static int stage_init(size_t slice) {
     if (!g_ctx.sev[b]) DDC_HIP(hipEventCreateWithFlags(&g_ctx.sev[b], hipEventDisableTiming));
     if (g_ctx.stage[b]) DDC_HIP(hipHostFree(g_ctx.stage[b]));
     g_ctx.stage[b] = nullptr;
-    DDC_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_ctx.stage[b]), cap, hipHostMallocDefault));
+    if (hipHostMalloc(reinterpret_cast<void**>(&g_ctx.stage[b]), cap, hipHostMallocDefault) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      g_ctx.stage[b] = nullptr;
+      *ok = false;
+      return DDC_OK;
+    }
   }
   g_ctx.stage_cap = cap;
   return DDC_OK;
@@ -265,12 +273,13 @@ static void host_copy2d(char* dst, size_t dpitch, const char* src, size_t spitch
 // host (pageable) -> device, stream-ordered on st; the caller synchronizes
 static int copy_h2d(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width,
                     size_t cols, hipStream_t st) {
-  if (width > STAGE_BYTES) {
+  const size_t slice = stage_slice(width * cols, width);
+  bool staged = width <= STAGE_BYTES;
+  if (staged) DDC_TRY(stage_init(slice, &staged));
+  if (!staged) {
     DDC_HIP(hipMemcpy2DAsync(dst, dpitch, src, spitch, width, cols, hipMemcpyHostToDevice, st));
     return DDC_OK;
   }
-  const size_t slice = stage_slice(width * cols, width);
-  DDC_TRY(stage_init(slice));
   const size_t per = slice / width;
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
@@ -291,13 +300,14 @@ static int copy_h2d(void* dst, size_t dpitch, const void* src, size_t spitch, si
 // device -> host (pageable); complete when it returns
 static int copy_d2h(void* dst, size_t dpitch, const void* src, size_t spitch, size_t width,
                     size_t cols, hipStream_t st) {
-  if (width > STAGE_BYTES) {
+  const size_t slice = stage_slice(width * cols, width);
+  bool staged = width <= STAGE_BYTES;
+  if (staged) DDC_TRY(stage_init(slice, &staged));
+  if (!staged) {
     DDC_HIP(hipMemcpy2DAsync(dst, dpitch, src, spitch, width, cols, hipMemcpyDeviceToHost, st));
     DDC_HIP(hipStreamSynchronize(st));
     return DDC_OK;
   }
-  const size_t slice = stage_slice(width * cols, width);
-  DDC_TRY(stage_init(slice));
   const size_t per = slice / width;
   const char* s = static_cast<const char*>(src);
   char* d = static_cast<char*>(dst);
@@ -333,11 +343,14 @@ static int copy_d2h(void* dst, size_t dpitch, const void* src, size_t spitch, si
 // matrix, this read included, takes 22 us (160 before).
 int host_read(void* dst, const void* src, size_t bytes, hipStream_t st) {
   if (bytes > MAIL_BYTES) return DDC_E_ARG;
-  if (!g_ctx.mail)
-    DDC_HIP(hipHostMalloc(reinterpret_cast<void**>(&g_ctx.mail), MAIL_BYTES, hipHostMallocDefault));
-  DDC_HIP(hipMemcpyAsync(g_ctx.mail, src, bytes, hipMemcpyDeviceToHost, st));
+  if (!g_ctx.mail && hipHostMalloc(reinterpret_cast<void**>(&g_ctx.mail), MAIL_BYTES,
+                                   hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    g_ctx.mail = nullptr;
+  }
+  DDC_HIP(hipMemcpyAsync(g_ctx.mail ? g_ctx.mail : dst, src, bytes, hipMemcpyDeviceToHost, st));
   DDC_HIP(hipStreamSynchronize(st));
-  memcpy(dst, g_ctx.mail, bytes);
+  if (g_ctx.mail) memcpy(dst, g_ctx.mail, bytes);
   return DDC_OK;
 }
 
