@@ -213,11 +213,6 @@ def right_gemv_bytes(m: int, n: int) -> int:
     return sum(8 * (m - k - 1) * (n - k - 1) for k in range(n - 2))
 
 
-def fused_gemv_bytes(m: int, n: int) -> int:
-    """Algorithmic bytes of the one-pass hook's launches: sum_{k<n-2} 8 (m-k)(n-k-1)."""
-    return sum(8 * (m - k) * (n - k - 1) for k in range(n - 2))
-
-
 def traffic_summary(m: int, n: int, kernel: str = "bd_left_gemv"):
     path = os.path.join(ROOT, "profiles", f"{kernel}_{m}x{n}_traffic.json")
     if not os.path.exists(path):
@@ -393,7 +388,7 @@ def backward_form(reps: int = 3) -> dict:
             "backward_ms": 1e3 * min(tb)}
 
 
-def pmc_pass(kernel: str, m: int, n: int, seed: int) -> int:
+def pmc_pass(kernel: str, m: int, n: int, seed: int, fused_launches: int = 0) -> int:
     """Workload for one rocprofv3 --pmc pass.  kernel "left" / "right": three
     1 GiB device copies (the calibration kernel of known traffic), then the
     left-GEMV (n-1) or right-GEMV (n-2) launches of one bidiagonalization
@@ -470,8 +465,10 @@ def pmc_pass(kernel: str, m: int, n: int, seed: int) -> int:
         print(f"pmc pass: {n - 1} left-GEMV launches, {m}x{n}", flush=True)
         ddcsvd.profile_left_gemv(A, n - 1, stream)
     elif kernel == "fused":
-        print(f"pmc pass: {n - 2} one-pass GEMV launches, {m}x{n}", flush=True)
-        ddcsvd.profile_fused_gemv(A, n - 2, stream)
+        # an SVD launches fewer where the rest of its steps runs in registers
+        steps = fused_launches or n - 2
+        print(f"pmc pass: {steps} one-pass GEMV launches, {m}x{n}", flush=True)
+        ddcsvd.profile_fused_gemv(A, steps, stream)
     else:
         print(f"pmc pass: {n - 2} right-GEMV launches, {m}x{n}", flush=True)
         ddcsvd.profile_right_gemv(A, n - 2, stream)
@@ -505,14 +502,21 @@ def summarize_pmc(kernel: str, fetch_dir: str, write_dir: str, m: int, n: int) -
         return per, names
 
     launches = n - 1 if kernel == "left" else n - 2
-    alg = {"left": left_gemv_bytes, "right": right_gemv_bytes,
-           "fused": fused_gemv_bytes}[kernel](m, n) / launches
+    arg = ""
+    if kernel == "fused":  # as many as the passes ran
+        per, names = load(fetch_dir, "FETCH_SIZE")
+        launches = sum(kname in names[k] for k in per) or launches
+        if launches != n - 2:
+            arg = f" --fused-launches {launches}"
+        alg = sum(8 * (m - k) * (n - k - 1) for k in range(launches)) / launches
+    else:
+        alg = {"left": left_gemv_bytes, "right": right_gemv_bytes}[kernel](m, n) / launches
     out = {"workload": f"the {launches} {kernel}-GEMV launches of one {m}x{n} N(0,1) "
                        f"bidiagonalization (svd_gpu_profile_{kernel}_gemv), seed 2",
            "commands": [f"rocprofv3 --pmc FETCH_SIZE -d {fetch_dir} -o run --output-format csv "
-                        f"-- python3 bench.py --pmc-pass {kernel} --m {m} --n {n}",
+                        f"-- python3 bench.py --pmc-pass {kernel} --m {m} --n {n}{arg}",
                         f"rocprofv3 --pmc WRITE_SIZE -d {write_dir} -o run --output-format csv "
-                        f"-- python3 bench.py --pmc-pass {kernel} --m {m} --n {n}",
+                        f"-- python3 bench.py --pmc-pass {kernel} --m {m} --n {n}{arg}",
                         f"python3 bench.py --summarize-pmc {kernel} {fetch_dir} {write_dir} "
                         f"--m {m} --n {n}"],
            "calibration": "bytes per counter unit = 1 GiB / the counter's mean over the three "
@@ -929,6 +933,8 @@ def main() -> int:
     ap.add_argument("--pmc-pass", choices=["left", "right", "fused", "gemm", "backtrans"],
                     help="workload of one rocprofv3 --pmc pass (copy calibration + one "
                          "GEMV kernel's launches, or the trailing-update GEMMs)")
+    ap.add_argument("--fused-launches", type=int, default=0,
+                    help="one-pass launches of --pmc-pass fused (default: all n - 2)")
     ap.add_argument("--summarize-pmc", nargs=3, metavar=("KERNEL", "FETCH_DIR", "WRITE_DIR"),
                     help="write the traffic summary of a GEMV kernel (left or right) from two "
                          "--pmc pass outputs")
@@ -960,7 +966,7 @@ def main() -> int:
     if args.summarize_pmc:
         return summarize_pmc(*args.summarize_pmc, args.m, args.n)
     if args.pmc_pass:
-        return pmc_pass(args.pmc_pass, args.m, args.n, args.seed)
+        return pmc_pass(args.pmc_pass, args.m, args.n, args.seed, args.fused_launches)
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported "
               f"(this build has no multi-GPU path)", file=sys.stderr)
