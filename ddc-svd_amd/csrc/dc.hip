@@ -30,7 +30,8 @@
 // merges: prep (one work-group per merge: rank-merge of the two
 // sorted child spectra, deflation, compaction), roots (one wave per root),
 // zhat (one wave per pole), rows (one wave per root: first/last rows of the
-// new singular vectors) and assemble (one work-group per merge).  The roots
+// new singular vectors) and assemble (one work-group per merge); depths of
+// ranges up to DC_SMALL do all five in one launch.  The roots
 // kernel gives a whole wave to each root: its lanes split the O(K) secular
 // sum, so the top merge of an n = 8192 problem fills the GPU.
 #include <algorithm>
@@ -41,6 +42,10 @@
 namespace ddc {
 
 constexpr double EPS = 2.220446049250313e-16;
+// Ranges up to here take one launch per depth (dc_small).  The stage at
+// n = 64, 256 and 1187, in us: 145, 218, 398 with none, 134, 200, 372 up to 8,
+// 140, 205, 371 up to 16, 179, 248, 385 up to 32.
+constexpr int DC_SMALL = 8;
 constexpr double TINY = 2.2250738585072014e-308;
 
 // A node of the tree: positions [off, off+N), split row off+K; a merge if
@@ -177,14 +182,11 @@ __device__ double group_max(double v, double* red) {
 // ---------------------------------------------------------------------------
 // prep: build the merged arrow, sort, deflate, compact.  One group per merge.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dc_prep(DcBufs B, int id0) {
+__device__ __forceinline__ void prep_merge(const DcBufs& B, int id, const DcMerge& M) {
   __shared__ double red[4];
   __shared__ int tmp[256];
   __shared__ double s_tol, s_scale;
   __shared__ int s_total;
-  const int id = id0 + blockIdx.x;
-  DcMerge M;
-  if (!dc_node(B.n, id, M) || M.N < 2) return;
   const int tid = threadIdx.x;
   const int off = M.off, N = M.N, K = M.K, N2 = N - K - 1;
   const double* s1 = B.sig + off;
@@ -399,22 +401,11 @@ __device__ __forceinline__ double wave_prod(double v) {
   return v;
 }
 
-// Work items: the grid covers the ids id0, id0 + 1, ... of one depth with
-// `groups` work-groups each, and a group of 256 threads takes 4 consecutive
-// items of its merge, one wave per item.
-#define DC_ITEM()                                                   \
-  const int id = id0 + (int)(blockIdx.x / (unsigned)groups);        \
-  DcMerge M;                                                        \
-  if (!dc_node(B.n, id, M) || M.N < 2) return;                      \
-  const int lane = threadIdx.x & 63;                                \
-  const int item = (int)(blockIdx.x % (unsigned)groups) * 4 +       \
-                   __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-
 // ---------------------------------------------------------------------------
 // roots: one wave per secular root
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dc_roots(DcBufs B, int id0, int groups) {
-  DC_ITEM();
+__device__ __forceinline__ void root_item(const DcBufs& B, int id, const DcMerge& M, int item,
+                                         int lane) {
   const DcMergeState st = B.ms[id];
   const int i = item;
   const int K = st.kept;
@@ -462,7 +453,8 @@ __global__ __launch_bounds__(256) void dc_roots(DcBufs B, int id0, int groups) {
   // bit by bisection was most of the time (up to 60 evaluations; now 4.3 on
   // average and 17 at most over random, graded and split spectra, with errors
   // no larger).  With the tree found on the device the stage went from 0.35 to
-  // 0.15 ms at n = 64 and from 1.0 to 0.40 ms at n = 1187.
+  // 0.15 ms at n = 64 and from 1.0 to 0.40 ms at n = 1187 (0.13 and 0.37 with
+  // dc_small).
   const double dO = d[o], dA = d[pa], dB = d[pb];
   double lo = 0.0, res = -1.0;
   for (int itn = 0; itn < 400; ++itn) {
@@ -519,8 +511,8 @@ __global__ __launch_bounds__(256) void dc_roots(DcBufs B, int id0, int groups) {
 //   * prod_{j<=k<K-1} (w_k^2 - d_j^2)/(d_{k+1}^2 - d_j^2)
 // with w_k - d_j = (d_{org(k)} - d_j) + tau_k.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dc_zhat(DcBufs B, int id0, int groups) {
-  DC_ITEM();
+__device__ __forceinline__ void zhat_item(const DcBufs& B, int id, const DcMerge& M, int item,
+                                         int lane) {
   const int K = B.ms[id].kept;
   const int j = item;
   if (j >= K) return;
@@ -547,8 +539,8 @@ __global__ __launch_bounds__(256) void dc_zhat(DcBufs B, int id0, int groups) {
 // ---------------------------------------------------------------------------
 // rows: one wave per root: first/last rows of the merged right vectors.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dc_rows(DcBufs B, int id0, int groups) {
-  DC_ITEM();
+__device__ __forceinline__ void row_item(const DcBufs& B, int id, const DcMerge& M, int item,
+                                         int lane) {
   const int K = B.ms[id].kept;
   const int i = item;
   if (i >= K) return;
@@ -586,10 +578,7 @@ __global__ __launch_bounds__(256) void dc_rows(DcBufs B, int id0, int groups) {
 // ---------------------------------------------------------------------------
 // assemble: merge the ascending roots with the ascending deflated values.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void dc_assemble(DcBufs B, int id0) {
-  const int id = id0 + blockIdx.x;
-  DcMerge M;
-  if (!dc_node(B.n, id, M) || M.N < 2) return;
+__device__ __forceinline__ void assemble_merge(const DcBufs& B, int id, const DcMerge& M) {
   const DcMergeState st = B.ms[id];
   const int off = M.off, N = M.N, K = st.kept, ND = N - K;
   const double* d = B.kd + off;
@@ -624,6 +613,66 @@ __global__ __launch_bounds__(256) void dc_assemble(DcBufs B, int id0) {
       B.lr[off + pos] = B.dL[off + q];
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// kernels
+// ---------------------------------------------------------------------------
+#define DC_MERGE()                       \
+  const int id = id0 + (int)blockIdx.x;  \
+  DcMerge M;                             \
+  if (!dc_node(B.n, id, M) || M.N < 2) return;
+
+// Work items: the grid covers the ids id0, id0 + 1, ... of one depth with
+// `groups` work-groups each, and a group of 256 threads takes 4 consecutive
+// items of its merge, one wave per item.
+#define DC_ITEM()                                                   \
+  const int id = id0 + (int)(blockIdx.x / (unsigned)groups);        \
+  DcMerge M;                                                        \
+  if (!dc_node(B.n, id, M) || M.N < 2) return;                      \
+  const int lane = threadIdx.x & 63;                                \
+  const int item = (int)(blockIdx.x % (unsigned)groups) * 4 +       \
+                   __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+__global__ __launch_bounds__(256) void dc_prep(DcBufs B, int id0) {
+  DC_MERGE();
+  prep_merge(B, id, M);
+}
+__global__ __launch_bounds__(256) void dc_roots(DcBufs B, int id0, int groups) {
+  DC_ITEM();
+  root_item(B, id, M, item, lane);
+}
+__global__ __launch_bounds__(256) void dc_zhat(DcBufs B, int id0, int groups) {
+  DC_ITEM();
+  zhat_item(B, id, M, item, lane);
+}
+__global__ __launch_bounds__(256) void dc_rows(DcBufs B, int id0, int groups) {
+  DC_ITEM();
+  row_item(B, id, M, item, lane);
+}
+__global__ __launch_bounds__(256) void dc_assemble(DcBufs B, int id0) {
+  DC_MERGE();
+  assemble_merge(B, id, M);
+}
+
+// The five in one launch, a work-group per merge, for depths of small ranges:
+// there a launch (4.7 us) costs more than the rounds of roots that each of
+// the four waves takes in turn.  Same functions, same results.
+__global__ __launch_bounds__(256) void dc_small(DcBufs B, int id0) {
+  DC_MERGE();
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  prep_merge(B, id, M);
+  __syncthreads();
+  for (int i = wave; i < M.N; i += 4) root_item(B, id, M, i, lane);
+  __syncthreads();
+  if (id != 1) {
+    for (int i = wave; i < M.N; i += 4) zhat_item(B, id, M, i, lane);
+    __syncthreads();
+    for (int i = wave; i < M.N; i += 4) row_item(B, id, M, i, lane);
+    __syncthreads();
+  }
+  assemble_merge(B, id, M);
 }
 
 // ---------------------------------------------------------------------------
@@ -698,6 +747,11 @@ int dc_run(int n, const double* a, const double* b, double* sigma, Arena& ws,
     const int id0 = 1 << p;                           // ids id0 .. 2 id0 - 1
     const int groups = (int)ceil_div((int64_t)(n >> p), 4);  // 4 items each
     const unsigned ni = (unsigned)id0 * (unsigned)groups;
+    if ((n >> p) <= DC_SMALL) {
+      hipLaunchKernelGGL(dc_small, dim3(id0), dim3(256), 0, st, B, id0);
+      DDC_LAUNCHED();
+      continue;
+    }
     hipLaunchKernelGGL(dc_prep, dim3(id0), dim3(256), 0, st, B, id0);
     DDC_LAUNCHED();
     hipLaunchKernelGGL(dc_roots, dim3(ni), dim3(256), 0, st, B, id0, groups);
