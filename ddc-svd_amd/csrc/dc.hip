@@ -11,11 +11,10 @@
 //  * relative deflation (|z_j| or pole gaps below 8 eps scale) with Givens
 //    rotations of the first/last rows, instead of the absolute thresholds
 //    1e-14/1e-20 (:143-144, :467);
-//  * each secular root is bracketed between its poles and found by bisection
-//    in the offset tau from the nearer pole (geometric while the bracket
-//    spans orders of magnitude), so sigma - d_j is formed without
-//    cancellation; no Newton steps that can jump to a neighbouring root
-//    (the reference's duplicate-root failure, :163-254);
+//  * each secular root is bracketed between its poles and found by
+//    interpolation, safeguarded by bisection, in the offset tau from the nearer
+//    pole, so sigma - d_j is formed without cancellation and no step can jump
+//    to a neighbouring root (the reference's duplicate-root failure, :163-254);
 //  * the first/last rows come from the Gu-Eisenstat z-hat (:445-465 uses a
 //    log-domain product with the same role), evaluated from the stored
 //    offsets.
