@@ -257,27 +257,53 @@ __device__ __forceinline__ bool jrot(T al, T be, T ga, T tol, T& c, T& s, T& t, 
 }
 
 // In FP64 the square roots and divisions of the general form (about 100
-// dependent instructions) are the longest part of a round.  The tangent only
-// steers convergence, so it comes from the hardware's reciprocals as they are
-// (about 2^-26: the dot product left behind is that factor of the old one);
-// the cosine is brought to full precision, so the rotation is orthogonal to
-// rounding.
+// dependent instructions) are the longest part of a round.  Here the same
+// angle comes from half the difference D of the squared norms,
+//     t = sign(D) g / (|D| + sqrt(D^2 + g^2)),
+// by the hardware's reciprocal and reciprocal square root (about 2^-26) and
+// one third-order correction each, to full precision:
+//  * D and g are taken relative to the larger norm, so that nothing over- or
+//    underflows for columns of any size (a reciprocal of a subnormal dot
+//    product is infinite), and the test for orthogonality relative to both;
+//    its scales and its bound need the norms alone, which are there before the
+//    dot product is.
+//  * The dot product that is left is the rounding of the old one.  With a
+//    tangent of 26 bits a column in the span of the others loses half as many
+//    digits per rotation: 20 to 26 sweeps on constant matrices and on ones of
+//    rank 2 and 3, now 11 to 18.
+//  * cos^2 + sin^2 must be 1 without bias, as every rotation scales its columns
+//    by it: the residual of the cosine's correction is formed from the exact
+//    product (two fused multiply-adds).  Over 200 matrices up to 256 x 256 the
+//    worst error of a singular value is 5.6e-15 of the largest (6.3e-14 with
+//    the tangent of 26 bits and the rounded product, 3.7e-14 with square roots
+//    and divisions).
+// A batch of 10,000 takes 85.4 ms (84.9 with the tangent of 26 bits).
+// off: 1 (the pair was not orthogonal to tol).
 template <>
 __device__ __forceinline__ bool jrot<double>(double al, double be, double ga, double tol,
                                              double& c, double& s, double& t, double& off) {
-  const double rel = fabs(ga) * __builtin_amdgcn_rsq(al) * __builtin_amdgcn_rsq(be);
-  if (!(al > 0.0) || !(be > 0.0) || !(rel > tol)) return false;
-  off = fmax(off, rel);
-  const double zeta = (be - al) * (0.5 * __builtin_amdgcn_rcp(ga));
-  const double az = fabs(zeta);
-  const double w = fma(az, az, 1.0);
-  const double tm = az > Num<double>::big ? 0.5 * __builtin_amdgcn_rcp(az)
-                                          : __builtin_amdgcn_rcp(az + w * __builtin_amdgcn_rsq(w));
-  t = zeta < 0.0 ? -tm : tm;
+  const int ea = __builtin_amdgcn_frexp_exp(al), eb = __builtin_amdgcn_frexp_exp(be);
+  const int ex = max(ea, eb), ee = ea + eb;
+  const double lim = tol * tol * __builtin_amdgcn_frexp_mant(al) *
+                     __builtin_amdgcn_frexp_mant(be) * ((ee & 1) ? 2.0 : 1.0);
+  const double D = ldexp(be, -ex - 1) - ldexp(al, -ex - 1);
+  const double gr = ldexp(ga, -(ee >> 1));
+  // (a zero norm, or a NaN: no rotation)
+  if (!(al > 0.0) || !(be > 0.0) || !(gr * gr > lim)) return false;
+  off = 1.0;
+  const double g = ldexp(ga, -ex);
+  const double h = fma(g, g, D * D);
+  const double z = __builtin_amdgcn_rsq(h);
+  const double p = h * z, e = fma(-p, z, 1.0);
+  const double den = fabs(D) + fma(p, e * fma(0.375, e, 0.5), p);
+  const double y = __builtin_amdgcn_rcp(den);
+  const double f = fma(-den, y, 1.0), t0 = g * y;
+  const double tm = fma(t0, fma(f, f, f), t0);
+  t = D < 0.0 ? -tm : tm;
   const double q = fma(t, t, 1.0);
-  const double z = __builtin_amdgcn_rsq(q);
-  const double e = fma(-q * z, z, 1.0);
-  c = fma(z * e, fma(0.375, e, 0.5), z);
+  const double x = __builtin_amdgcn_rsq(q);
+  const double w = q * x, r = fma(-fma(q, x, -w), x, fma(-w, x, 1.0));
+  c = fma(x * r, fma(0.375, r, 0.5), x);
   s = c * t;
   return true;
 }
