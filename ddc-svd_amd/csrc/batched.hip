@@ -35,10 +35,11 @@
 //    zero norm are completed to an orthonormal basis by Gram-Schmidt on unit
 //    vectors.
 //
-// Two tunables are picked by measurement (svd_gpu_batched_tune): the kernel
-// variant (block width per row class, which also sets the register budget
-// and so the waves of a workgroup; FP64 only) and the cooperation threshold
-// coop_nt.
+// The kernel variant (block width per row class, which also sets the register
+// budget and so the waves of a workgroup) decides the order of the rotations
+// and with it the last digits of the results: it is picked by the sizes of the
+// batch (bj_variant).  The cooperation threshold coop_nt changes no bit, and is
+// picked by measurement (svd_gpu_batched_tune).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -316,20 +317,33 @@ struct Block {
   T v[2 * B][RV];
 };
 
+// x y + z.  In FP64 fused wherever it is inlined: left to the compiler, the
+// copies of one expression in the sweeps of a workgroup and of a wave alone
+// round differently.
+template <typename T>
+__device__ __forceinline__ T madd(T x, T y, T z) {
+  if constexpr (sizeof(T) == 8) return fma(x, y, z);
+  else return x * y + z;
+}
+
+template <typename T>
+__device__ __forceinline__ void turn(T& x, T& y, T c, T s) {
+  const T u = x, v = y;
+  if constexpr (sizeof(T) == 8) {
+    x = fma(c, u, -(s * v));
+    y = fma(s, u, c * v);
+  } else {
+    x = c * u - s * v;
+    y = s * u + c * v;
+  }
+}
+
 template <typename T, int B, int R, int RV>
 __device__ __forceinline__ void rotate_cols(Block<T, B, R, RV>& k, int p, int q, T c, T s) {
 #pragma unroll
-  for (int e = 0; e < R; ++e) {
-    const T x = k.a[p][e], y = k.a[q][e];
-    k.a[p][e] = c * x - s * y;
-    k.a[q][e] = s * x + c * y;
-  }
+  for (int e = 0; e < R; ++e) turn(k.a[p][e], k.a[q][e], c, s);
 #pragma unroll
-  for (int e = 0; e < RV; ++e) {
-    const T x = k.v[p][e], y = k.v[q][e];
-    k.v[p][e] = c * x - s * y;
-    k.v[q][e] = s * x + c * y;
-  }
+  for (int e = 0; e < RV; ++e) turn(k.v[p][e], k.v[q][e], c, s);
 }
 
 // Cross round S of a block pair: B disjoint rotations, column i of block I
@@ -346,7 +360,7 @@ __device__ __forceinline__ void cross_round(Block<T, B, R, RV>& k, T& al, T& be,
   for (int i = 0; i < B; ++i) {
     T d = T(0);
 #pragma unroll
-    for (int e = 0; e < R; ++e) d += k.a[i][e] * k.a[B + (i + S) % B][e];
+    for (int e = 0; e < R; ++e) d = madd(k.a[i][e], k.a[B + (i + S) % B][e], d);
     g[i] = d;
   }
   const T gl = lane_scatter<T, B>(g);
@@ -391,8 +405,8 @@ __device__ __forceinline__ void intra_round(Block<T, B, R, RV>& k, T& nrm, bool 
     if (i < H ? enI : enJ) {
 #pragma unroll
       for (int e = 0; e < R; ++e)
-        d += k.a[i / H * B + circle<B, S>(i % H)][e] *
-             k.a[i / H * B + circle<B, S>(B - 1 - i % H)][e];
+        d = madd(k.a[i / H * B + circle<B, S>(i % H)][e],
+                 k.a[i / H * B + circle<B, S>(B - 1 - i % H)][e], d);
     }
     g[i] = d;
   }
@@ -484,7 +498,7 @@ __device__ __forceinline__ T col_norms(const Block<T, B, R, RV>& k) {
     for (int c = 0; c < 2 * B; ++c) {
       T s = T(0);
 #pragma unroll
-      for (int e = 0; e < R; ++e) s += k.a[c][e] * k.a[c][e];
+      for (int e = 0; e < R; ++e) s = madd(k.a[c][e], k.a[c][e], s);
       part[c] = s;
     }
     return lane_scatter<T, 2 * B>(part);
@@ -679,6 +693,49 @@ __device__ __forceinline__ int bj_sweeps_super(T* W, T* WV, int mt, int nt, Team
   return -1;
 }
 
+// The same sweeps by a wave alone, one block pair after another.  The pairs of
+// a round are disjoint, so every column sees the same rotations in the same
+// order as with NW waves: which matrices a workgroup takes together is a
+// question of time alone, and the results are the same bit for bit.
+template <typename T, int B, int R, int RV, int NW>
+__device__ __forceinline__ int bj_sweeps_alone(T* W, T* WV, int mt, int nt, Team t) {
+  const T tol = Num<T>::eps * sqrt(T(mt));
+  mt = __builtin_amdgcn_readfirstlane(mt);
+  nt = __builtin_amdgcn_readfirstlane(nt);
+  const int nb = (nt + B - 1) / B;
+  const int ns = (nb + NW - 1) / NW, q = (nb + ns - 1) / ns;
+  const int qe = q + (q & 1), hq = qe / 2;
+  const int inside = max(qe - 1, 1);  // rounds inside the super-blocks
+  for (int sw = 0; sw < BJ_MAXSWEEP; ++sw) {
+    T off = T(0);
+    int S = 0, U = 1, d = 0;  // across: block w of S with block w + d of U
+    for (int r = 0; r < inside || S + 1 < ns; ++r) {
+      const bool in = r < inside;
+      for (int i = 0; i < (in ? ns * hq : q); ++i) {
+        int I = S * q + i, J = U * q + (i + d < q ? i + d : i + d - q);
+        bool alone = false;
+        if (in) {
+          const int s = i / hq, pi = i - s * hq;
+          const int x = rr_p(qe, r, pi), y = rr_q(qe, r, pi);
+          I = s * q + min(x, y);
+          J = s * q + max(x, y);
+          alone = max(x, y) >= q || J >= nb;
+        }
+        if (I >= nb || (J >= nb && !alone) || (alone && r != 0)) continue;
+        off = fmax(off, block_step<T, B, R, RV>(W, WV, mt, nt, I * B, alone ? -1 : J * B, r == 0,
+                                                r == 0 && !alone, tol));
+      }
+      t.sync();
+      if (!in && ++d == q) {
+        d = 0;
+        if (++U == ns) U = ++S + 1;
+      }
+    }
+    if (!(wmax(off) > tol)) return sw + 1;
+  }
+  return -1;
+}
+
 // Copies A (transposed when wide) into W scaled by a power of two so that
 // max |a| is in [0.5, 1), and sets WV = I.  Returns the scale.
 template <typename T>
@@ -801,7 +858,7 @@ __device__ __forceinline__ int64_t uni64(int64_t x) {
   return ((int64_t)hi << 32) | (int64_t)(unsigned)lo;
 }
 
-template <typename T, int B, int R, int RV>
+template <typename T, int B, int R, int RV, int NW>
 __device__ __forceinline__ void bj_matrix(const BatchItem& it, const BjArgs<T>& g, int k,
                                           Team t, T* sig, int* rk, T* red, T* xch) {
   const int mt = it.m > it.n ? it.m : it.n, nt = it.m > it.n ? it.n : it.m;
@@ -809,8 +866,9 @@ __device__ __forceinline__ void bj_matrix(const BatchItem& it, const BjArgs<T>& 
   T* WV = (T*)uni64((int64_t)(g.WV + it.wv));
   const T scale = bj_load(it, g.A, W, WV, mt, nt, t, red);
   int sweeps;
-  if (sizeof(T) == 8 && t.nw > 1)
-    sweeps = bj_sweeps_super<T, B, R, RV>(W, WV, mt, nt, t, red, xch);
+  if constexpr (sizeof(T) == 8)
+    sweeps = t.nw > 1 ? bj_sweeps_super<T, B, R, RV>(W, WV, mt, nt, t, red, xch)
+                      : bj_sweeps_alone<T, B, R, RV, NW>(W, WV, mt, nt, t);
   else
     sweeps = bj_sweeps<T, B, R, RV>(W, WV, mt, nt, t, red);
   bj_finish(it, g, W, WV, mt, nt, scale, sig, rk, t);
@@ -887,7 +945,7 @@ __global__ __launch_bounds__(256 * MINW, MINW) void bj_kernel(BjArgs<T> g) {
     const int R = (mt + 63) / 64, RV = (nt + 63) / 64;
 #define BJ_CASE(R_, RV_)                                                  \
   if (R == R_ && RV == RV_) {                                             \
-    bj_matrix<T, (R_ <= 2 ? B12 : B34), R_, RV_>(it, g, k, t, sg, rkk, rd, xch); \
+    bj_matrix<T, (R_ <= 2 ? B12 : B34), R_, RV_, WGW>(it, g, k, t, sg, rkk, rd, xch); \
     continue;                                                             \
   }
     BJ_CASE(1, 1)
@@ -931,10 +989,9 @@ static const BjVariant kVariants[] = {
 };
 #undef BJ_VARIANT
 constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
-static const int kWgsPerCu[] = {1};
-// (one workgroup holds all the waves a CU can)
-// first entry: the threshold used while the variants are compared
-static const int kCoopNt[] = {32, 1, 8, 16, 64, 96, 128, 192, BJ_MAXDIM + 1};
+// thresholds that the tuner times, the first one and those below it, then those
+// above it in rising order
+static const int kCoopNt[] = {32, 1, 8, 12, 16, 20, 24, 40, 48, 64, 96, 128, BJ_MAXDIM + 1};
 
 // A launch configuration: kernel variant, resident workgroups per CU, and
 // the smallest min(m, n) a whole workgroup factors together.
@@ -953,9 +1010,9 @@ static int bj_launch(const BjConfig& c, int cus, BjArgs<T> a, hipStream_t st) {
   return DDC_OK;
 }
 
-// tuned configurations by (dtype, log2 count, log2 work)
+// tuned thresholds by (dtype, variant, log2 count, log2 work)
 static std::mutex g_tune_mu;
-static std::map<std::tuple<int, int, int>, BjConfig> g_tune_cache;
+static std::map<std::tuple<int, int, int, int>, int> g_tune_cache;
 
 }  // namespace ddc
 
@@ -1010,16 +1067,12 @@ static int bj_enqueue(svd_gpu_batch* p, const BjConfig& c, const void* dA, void*
   return bj_launch<float>(c, p->cus, bj_args<float>(p, dA, dS, dU, dV, info), st);
 }
 
-static std::tuple<int, int, int> tune_key(const svd_gpu_batch* p) {
-  return {p->dtype, (int)std::lround(std::log2((double)p->count)),
-          (int)std::lround(std::log2(p->work + 1.0))};
-}
-
-// Milliseconds of one launch of configuration c on the whole batch (best of 2).
+// Milliseconds of one launch of configuration c on the whole batch (best of 2;
+// one alone where it is far from best, the time to beat).
 static int bj_time(svd_gpu_batch* p, const BjConfig& c, const void* dA, void* dS, void* dU,
-                   void* dV, hipStream_t st, hipEvent_t e0, hipEvent_t e1, float& ms) {
+                   void* dV, hipStream_t st, hipEvent_t e0, hipEvent_t e1, float best, float& ms) {
   ms = 1e30f;
-  for (int rep = 0; rep < 2; ++rep) {
+  for (int rep = 0; rep < 2 && !(rep > 0 && ms > 1.2f * best); ++rep) {
     DDC_HIP(hipEventRecord(e0, st));
     DDC_TRY(bj_enqueue(p, c, dA, dS, dU, dV, nullptr, st));
     DDC_HIP(hipEventRecord(e1, st));
@@ -1031,27 +1084,52 @@ static int bj_time(svd_gpu_batch* p, const BjConfig& c, const void* dA, void* dS
   return DDC_OK;
 }
 
-// The variant of an FP32 batch, by its sizes: the results depend on the block
-// width in their last digits, and the two widths that come into question are
-// within 2% of each other wherever the largest matrix decides the time, so a
-// timing would pick one or the other from run to run.  Blocks of 4 throughout
-// are the faster ones (by 2%: 17.9 against 18.3 ms for 2,500 matrices up to
-// 256) for batches that are mostly a few matrices above 224 rows; blocks of 8
-// up to 128 rows everywhere else (13.1 against 17.0 ms for 10,000 up to 128).
-static int bj_variant_f32(const svd_gpu_batch* p) {
-  int rows = 0;
+// The variant of a batch, 0 (blocks of 8 up to 128 rows, of 4 beyond) or 1
+// (blocks of 4), by its sizes: a timing would pick one or the other from run to
+// run where they are close, and the results differ in their last digits (in
+// vectors of close values by more).  The narrower ones have more waves at work
+// on a matrix, the wider ones pass over it half as often.  ms, 8 | 4 wide, each
+// at its best threshold:
+//  * FP64, load = work / (CUs x work of the largest):
+//      up to 40 columns, few matrices: 24 x 24, 256 of them, 0.29 | 0.18, 512
+//      0.50 | 0.33, 1024 0.52 | 0.64; 800 up to 40 x 40 (load 0.43) 0.47 | 0.39,
+//      1600 (0.86) 0.61 | 0.67;
+//      up to 8 columns, which one block of 8 leaves no other: 2048 of 8 x 8
+//      0.13 | 0.10, 3000 of 128 x 8 0.21 | 0.16;
+//      more columns: 200 of 128 x 128 2.7 | 3.5, 2000 20 | 26, 10,000 up to 128
+//      15.5 | 17.4, up to 256 84.3 | 85.3, 300 up to 64 0.60 | 0.61; the other
+//      way by at most a tenth (1600 up to 96 2.63 | 2.41, 800 up to 64
+//      0.70 | 0.65);
+//      all of more than 128 rows: one width and one result, 0 to 5% in favour of
+//      the kernel that holds it alone (8000 of 200 x 8 0.482 | 0.458).
+//  * FP32: blocks of 8 wherever the matrices of up to 128 rows count (10,000 up
+//    to 128 13.3 | 15.7, 2000 of 128 x 128 16.6 | 22.2).  Where one of more than
+//    224 rows outlasts the others the two are within 1% (150 up to 256
+//    12.1 | 12.0, 600 12.7 | 12.8, 2,500 19.6 | 19.5), so the line between them
+//    costs nothing wherever it lies.
+static int bj_variant(const svd_gpu_batch* p) {
+  int rows = 0, least = BJ_MAXDIM, cols = 0;
   double most = 0.0;
   for (int k = 0; k < p->count; ++k) {
     const int mt = std::max(p->m[k], p->n[k]), nt = std::min(p->m[k], p->n[k]);
     rows = std::max(rows, mt);
+    least = std::min(least, mt);
+    cols = std::max(cols, nt);
     most = std::max(most, (double)nt * nt * mt);
   }
-  return rows > 224 && p->work < 350.0 * most ? 1 : 0;
+  if (p->dtype == SVD_GPU_F32) return rows > 224 && p->work < 350.0 * most ? 1 : 0;
+  const bool few = p->count <= 2 * p->cus || p->work < 0.6 * p->cus * most;
+  return cols <= 8 || least > 128 || (cols <= 40 && few) ? 1 : 0;
 }
 
-// The autotuner: times the variants (FP64; see bj_variant_f32) with a middle
-// cooperation threshold, then the thresholds for the best one, each on the
-// whole batch.  (A half-size sample was tried: it keeps the largest
+static std::tuple<int, int, int, int> tune_key(const svd_gpu_batch* p) {
+  return {p->dtype, bj_variant(p), (int)std::lround(std::log2((double)p->count)),
+          (int)std::lround(std::log2(p->work + 1.0))};
+}
+
+// The autotuner: times the thresholds, each on the whole batch, but those that
+// split it as an earlier one does and, once a larger one takes twice the best
+// time, the ones beyond.  (A half-size sample was tried: it keeps the largest
 // matrices, whose latency floors the makespan, but only half of the bulk,
 // and ranked configurations 25% apart in the wrong order.)
 static int bj_tune(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* dV,
@@ -1063,32 +1141,24 @@ static int bj_tune(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* d
     return DDC_E_HIP;
   }
   float best = 1e30f;
-  BjConfig bc;
+  BjConfig bc, c;
+  c.variant = bj_variant(p);
+  c.wgs = 1;  // one workgroup holds all the waves a CU can
   int rc = DDC_OK;
-  const int only = p->dtype == SVD_GPU_F32 ? bj_variant_f32(p) : -1;
-  for (int v = 0; v < kNumVariants && !rc; ++v)
-    for (int wg : kWgsPerCu) {
-      if (only >= 0 && v != only) continue;
-      BjConfig c;
-      c.variant = v;
-      c.wgs = wg;
-      c.coop_nt = kCoopNt[0];
-      float ms;
-      if ((rc = bj_time(p, c, dA, dS, dU, dV, st, e0, e1, ms))) break;
-      if (ms < best) {
-        best = ms;
-        bc = c;
-      }
-    }
+  std::vector<int> seen;  // matrices taken by whole workgroups
   for (int ct : kCoopNt) {
-    if (rc || ct == kCoopNt[0]) continue;
-    BjConfig c = bc;
+    int whole = 0;
+    for (int k = 0; k < p->count; ++k) whole += std::min(p->m[k], p->n[k]) >= ct;
+    if (std::find(seen.begin(), seen.end(), whole) != seen.end()) continue;
+    seen.push_back(whole);
     c.coop_nt = ct;
     float ms;
-    if ((rc = bj_time(p, c, dA, dS, dU, dV, st, e0, e1, ms))) break;
+    if ((rc = bj_time(p, c, dA, dS, dU, dV, st, e0, e1, best, ms))) break;
     if (ms < best) {
       best = ms;
       bc = c;
+    } else if (ct > kCoopNt[0] && ms > 2.0f * best) {
+      break;
     }
   }
   (void)hipEventDestroy(e0);
@@ -1096,7 +1166,7 @@ static int bj_tune(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* d
   if (rc) return rc;
   p->cfg = bc;
   std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune_cache[tune_key(p)] = bc;
+  g_tune_cache[tune_key(p)] = bc.coop_nt;
   return DDC_OK;
 }
 
@@ -1202,8 +1272,9 @@ static int bj_plan(svd_gpu_batch* p, int count, const int* m, const int* n, int 
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto f = g_tune_cache.find(tune_key(p));
     if (f != g_tune_cache.end()) {
-      p->cfg = f->second;
-      if (dtype == SVD_GPU_F32) p->cfg.variant = bj_variant_f32(p);
+      p->cfg.variant = bj_variant(p);
+      p->cfg.wgs = 1;
+      p->cfg.coop_nt = f->second;
     }
   }
   return DDC_OK;

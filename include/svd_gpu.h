@@ -199,9 +199,10 @@ int svd_gpu_batched_offsets(const svd_gpu_batch *plan, long long *offA,
  */
 int svd_gpu_batched_run(svd_gpu_batch *plan, const void *dA, void *dsigma,
                         void *dU, void *dV, int *dinfo, void *stream);
-/* Times the kernel variants, launch sizes and cooperation thresholds on the
- * whole batch (the result is also remembered for later plans of similar
- * batches); writes the outputs.  Synchronous. */
+/* Times the cooperation thresholds on the whole batch (the result is also
+ * remembered for later plans of similar batches); writes the outputs.  The
+ * threshold does not change the results; the kernel variant, which does in the
+ * last digits, goes by the sizes of the batch.  Synchronous. */
 int svd_gpu_batched_tune(svd_gpu_batch *plan, const void *dA, void *dsigma,
                          void *dU, void *dV, void *stream);
 /* Chosen configuration: kernel variant, resident workgroups per CU,
