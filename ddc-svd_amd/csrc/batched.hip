@@ -1145,12 +1145,12 @@ static int bj_tune(svd_gpu_batch* p, const void* dA, void* dS, void* dU, void* d
   c.variant = bj_variant(p);
   c.wgs = 1;  // one workgroup holds all the waves a CU can
   int rc = DDC_OK;
-  std::vector<int> seen;  // matrices taken by whole workgroups
+  int seen[sizeof(kCoopNt) / sizeof(kCoopNt[0])], ns = 0;  // matrices taken by whole workgroups
   for (int ct : kCoopNt) {
     int whole = 0;
     for (int k = 0; k < p->count; ++k) whole += std::min(p->m[k], p->n[k]) >= ct;
-    if (std::find(seen.begin(), seen.end(), whole) != seen.end()) continue;
-    seen.push_back(whole);
+    if (std::find(seen, seen + ns, whole) != seen + ns) continue;
+    seen[ns++] = whole;
     c.coop_nt = ct;
     float ms;
     if ((rc = bj_time(p, c, dA, dS, dU, dV, st, e0, e1, best, ms))) break;
