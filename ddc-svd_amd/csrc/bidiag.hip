@@ -1394,8 +1394,11 @@ static bool fused_gemv_on() {
 
 template <typename TS>
 static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* beta, int upd,
-                        Arena& ws, hipStream_t st) {
+                        Arena& ws, hipStream_t st, BidiagForm* form) {
   if (m < 1 || n < 1 || lda < m || (lda % 2) != 0) return DDC_E_ARG;
+  BidiagForm lib;
+  if (!form) form = &lib;
+  form->stopped = -1;
   BidiagBufs d = bidiag_dims(m, n, lda);
   StepArgs<TS> a;
   a.m = m;
@@ -1446,7 +1449,7 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
            n - kk - 1 <= FG_GMAX * FG_MAXCOL;
   };
   // columns from this panel boundary on fit the register files (resident.hip)
-  int res_k = fused_gemv_on() ? resident_first<TS>(m, n, NB) : -1;
+  int res_k = fused_gemv_on() && form->resident ? resident_first<TS>(m, n, NB) : -1;
   // the panel operands' padding and the first column's norm: not needed where
   // the steps run in registers from the first one on (four launches)
   auto begin = [&](int k) {
@@ -1473,11 +1476,12 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
     fusedL = 0;
     if (k == res_k) {
       int done = 0;
-      DDC_TRY(resident_run<TS>(m, n, A, lda, alpha, beta, k, NB, ws, st, &done));
+      DDC_TRY(resident_run<TS>(m, n, A, lda, alpha, beta, k, NB, ws, st, &done, form->absent));
       if (done >= mn) break;
       // the work-groups found no room beside other work: the rest below,
       // from panel boundary `done` (resident_run is not tried again)
       res_k = -1;
+      form->stopped = done;
       k = done - 1;
       DDC_TRY(begin(done));
       continue;
@@ -1597,8 +1601,8 @@ static int bidiag_drive(int m, int n, TS* A, int lda, double* alpha, double* bet
 }
 
 int bidiag_run(int m, int n, double* A, int lda, double* alpha, double* beta, Arena& ws,
-               hipStream_t st) {
-  return bidiag_drive<double>(m, n, A, lda, alpha, beta, 0, ws, st);
+               hipStream_t st, BidiagForm* form) {
+  return bidiag_drive<double>(m, n, A, lda, alpha, beta, 0, ws, st, form);
 }
 
 // Measurement: `steps` left-GEMV launches, at column steps k = 0..steps-1,
@@ -1763,9 +1767,9 @@ int bidiag_right_gemv_only(int m, int n, double* A, int lda, double* alpha, int 
 }
 
 int bidiag_run_f32(int m, int n, float* A, int lda, double* alpha, double* beta, int upd,
-                   Arena& ws, hipStream_t st) {
+                   Arena& ws, hipStream_t st, BidiagForm* form) {
   if (upd != UPD_F32 && upd != UPD_BF16X3 && upd != UPD_BF16) return DDC_E_ARG;
-  return bidiag_drive<float>(m, n, A, lda, alpha, beta, upd, ws, st);
+  return bidiag_drive<float>(m, n, A, lda, alpha, beta, upd, ws, st, form);
 }
 
 }  // namespace ddc

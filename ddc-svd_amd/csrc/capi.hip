@@ -905,6 +905,45 @@ static int backward_dev(int m, int n, const double* U, int ldu, const double* si
 }
 
 // host buffers: A (m x n, reflectors as bidiag_gpu leaves them) -> Q
+// The bidiagonalization alone by a given form, for the tests: A (m x n, host,
+// FP64 or FP32 storage) is replaced by the reflectors; *ms: its time on the
+// device.
+template <typename TS>
+static int test_bidiag(int m, int n, TS* A, double* alpha, double* beta, BidiagForm* form,
+                       float* ms) {
+  DDC_TRY(check_dims(m, n));
+  DDC_TRY(ctx_init());
+  hipStream_t st = g_ctx.st;
+  const int lda_p = (int)round_up(m, 16), mn = std::min(m, n), nbeta = m >= n ? n - 1 : m;
+  ArenaPlan plan;
+  plan.add<TS>((size_t)lda_p * n);
+  plan.add<double>(n);
+  plan.add<double>(n);
+  if constexpr (sizeof(TS) == 8) bidiag_plan(plan, m, n, lda_p);
+  else bidiag_plan_f32(plan, m, n, lda_p, UPD_F32);
+  Arena ws;
+  DDC_TRY(arena_get(plan.bytes, ws, st));
+  TS* Ap = ws.take<TS>((size_t)lda_p * n);
+  double* da = ws.take<double>(n);
+  double* db = ws.take<double>(n);
+  if (!db) return DDC_E_NOMEM;
+  DDC_HIP(hipMemsetAsync(Ap, 0, sizeof(TS) * (size_t)lda_p * n, st));
+  const size_t D = sizeof(TS);
+  DDC_TRY(copy_h2d(Ap, D * lda_p, A, D * m, D * m, n, st));
+  Timer tm;
+  DDC_TRY(tm.create(st));
+  DDC_TRY(tm.mark());
+  if constexpr (sizeof(TS) == 8) DDC_TRY(bidiag_run(m, n, Ap, lda_p, da, db, ws, st, form));
+  else DDC_TRY(bidiag_run_f32(m, n, Ap, lda_p, da, db, UPD_F32, ws, st, form));
+  DDC_TRY(tm.mark());
+  DDC_TRY(copy_d2h(A, D * m, Ap, D * lda_p, D * m, n, st));
+  const size_t wa = sizeof(double) * mn, wb = sizeof(double) * nbeta;
+  DDC_TRY(copy_d2h(alpha, wa, da, wa, wa, 1, st));
+  if (nbeta > 0) DDC_TRY(copy_d2h(beta, wb, db, wb, wb, 1, st));
+  DDC_HIP(hipEventElapsedTime(ms, tm.ev[0], tm.ev[1]));
+  return DDC_OK;
+}
+
 static int form_host(bool left, int m, int n, const double* A, double* Q) {
   DDC_TRY(check_dims(m, n));
   if (m < n) {
@@ -1112,5 +1151,21 @@ int svd_gpu_dgemm(char transa, char transb, int M, int N, int K, double alpha, c
 }
 
 const char* svd_gpu_last_error(void) { return g_err; }
+
+// The entry points below are the tests' own (not declared in svd_gpu.h).
+
+// resident: 0 the panel kernels throughout; absent: BidiagForm.
+int ddc_test_bidiag(int m, int n, void* A, int f32, double* alpha, double* beta, int resident,
+                    int absent, int* stopped, float* ms) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_err[0] = 0;
+  BidiagForm form;
+  form.resident = resident != 0;
+  form.absent = absent;
+  const int rc = f32 ? test_bidiag(m, n, static_cast<float*>(A), alpha, beta, &form, ms)
+                     : test_bidiag(m, n, static_cast<double*>(A), alpha, beta, &form, ms);
+  *stopped = form.stopped;
+  return rc;
+}
 
 }  // extern "C"

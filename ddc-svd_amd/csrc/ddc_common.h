@@ -101,8 +101,15 @@ int bidiag_fused_gemv_only(int m, int n, double* A, int lda, double* alpha, int 
 // Measurement: `steps` right-GEMV launches (after one left GEMV at k = 0).
 int bidiag_right_gemv_only(int m, int n, double* A, int lda, double* alpha, int steps,
                            Arena& ws, hipStream_t st);
+// How the column steps are done: by default in registers from where the rest
+// fits (the library's calls).  The other settings are the tests'.
+struct BidiagForm {
+  bool resident = true;  // false: by the panel kernels throughout
+  int absent = -1;       // launch of resident_run that waits for one work-group too many
+  int stopped = -1;      // out: the step from which its launches gave up
+};
 int bidiag_run(int m, int n, double* A, int lda, double* alpha, double* beta,
-               Arena& ws, hipStream_t st);
+               Arena& ws, hipStream_t st, BidiagForm* form = nullptr);
 
 // The same with the matrix and its reflectors stored in FP32 (vector
 // arithmetic stays FP64) and the blocked trailing update in reduced
@@ -112,19 +119,19 @@ int bidiag_run(int m, int n, double* A, int lda, double* alpha, double* beta,
 enum { UPD_F32 = 1, UPD_BF16X3 = 2, UPD_BF16 = 3 };
 void bidiag_plan_f32(ArenaPlan& p, int m, int n, int lda, int upd);
 int bidiag_run_f32(int m, int n, float* A, int lda, double* alpha, double* beta, int upd,
-                   Arena& ws, hipStream_t st);
+                   Arena& ws, hipStream_t st, BidiagForm* form = nullptr);
 
 // The column steps from k0 on with the matrix in registers (resident.hip):
 // for what is left of the matrix at k0 >= resident_first(), itself a multiple
 // of align (or -1: never).  *done: steps completed, a multiple of align or
 // min(m, n); less than min(m, n) where the work-groups found no room, A being
-// updated up to there.  Synchronizes st.
+// updated up to there.  absent: BidiagForm.  Synchronizes st.
 template <typename TS>
 int resident_first(int m, int n, int align);
 void resident_plan(ArenaPlan& p);
 template <typename TS>
 int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int k0, int align,
-                 Arena& ws, hipStream_t st, int* done);
+                 Arena& ws, hipStream_t st, int* done, int absent);
 
 // Mixed-precision SVD of the n x n FP64 matrix A (device pointers): FP32
 // bidiagonalization with update mode upd, FP64 bidiagonal solve, FP32

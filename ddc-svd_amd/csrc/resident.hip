@@ -110,6 +110,7 @@ constexpr unsigned RS_GO = 1, RS_STOP = 2, RS_FAILED = 1000;
 template <typename TS>
 struct ResArgs {
   int m, n, lda, k0, k1, idx;
+  unsigned groups;  // work-groups that the launch waits for
   TS* A;
   double* alpha;
   double* beta;
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(RS_T, 1) void bd_resident(ResArgs<TS> g) {
       unsigned* arrived = g.sync + 16 * g.idx;
       unsigned* state = arrived + 1;
       if (go) {
-        if (atomicAdd(arrived, 1u) + 1 == (unsigned)(PR * PC)) atomicCAS(state, 0u, RS_GO);
+        if (atomicAdd(arrived, 1u) + 1 == g.groups) atomicCAS(state, 0u, RS_GO);
         for (int i = 0; i < RS_RDV && take(state) == 0; ++i) __builtin_amdgcn_s_sleep(8);
         // all decide alike: whoever writes the state first decides
         atomicCAS(state, 0u, RS_STOP);
@@ -776,7 +777,7 @@ __global__ __launch_bounds__(1024) void rs_clear(unsigned* sync, double* beta, i
 
 template <typename TS>
 int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int k0, int align,
-                 Arena& ws, hipStream_t st, int* done) {
+                 Arena& ws, hipStream_t st, int* done, int absent) {
   int cnt;
   const ResShape<TS>* tab = res_shapes<TS>(&cnt);
   int64_t mx = 0;
@@ -809,6 +810,7 @@ int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int 
     a.k0 = k;
     a.k1 = k1;
     a.idx = nl;
+    a.groups = (unsigned)(s.pr * s.pc) + (nl == absent ? 1u : 0u);
     a.A = A;
     a.alpha = alpha;
     a.beta = beta;
@@ -837,8 +839,8 @@ int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int 
 template int resident_first<double>(int, int, int);
 template int resident_first<float>(int, int, int);
 template int resident_run<double>(int, int, double*, int, double*, double*, int, int, Arena&,
-                                  hipStream_t, int*);
+                                  hipStream_t, int*, int);
 template int resident_run<float>(int, int, float*, int, double*, double*, int, int, Arena&,
-                                 hipStream_t, int*);
+                                 hipStream_t, int*, int);
 
 }  // namespace ddc
