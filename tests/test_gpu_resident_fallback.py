@@ -79,6 +79,19 @@ def test_each_launch_in_turn_gives_up(ddcsvd, shape, dtype):
     _check(ddcsvd, A, out, dtype)
 
 
+@pytest.mark.parametrize("shape", [(400, 200), (700, 600)], ids=lambda s: f"{s[0]}x{s[1]}")
+def test_giving_up_is_quick(ddcsvd, shape):
+    """The wait is bound to about 1 ms: the call takes that and the panel kernels'
+    time, 10 ms left for everything else (the best of three).  400 x 200: the
+    work-groups of one XCD, 700 x 600: of all."""
+    A = gen.normal_matrix(*shape, seed=1)
+    gpu_case(f"resident launch 0 of {shape[0]}x{shape[1]} gives up, timed")
+    extra = min(_bidiag(ddcsvd, A, np.float64, absent=0)[2]
+                - _bidiag(ddcsvd, A, np.float64, resident=0)[2] for _ in range(3))
+    print(f"[giving-up] {shape}: {extra:.2f} ms beyond the panel kernels", flush=True)
+    assert extra <= 10.0
+
+
 # (70, 66): the panel boundary k = 64 is column n - 2; (2500, 200), (4200, 130):
 # several chunks of rows in the GEMVs; (33, 33), (65, 90): one step past a panel
 @pytest.mark.parametrize("dtype", [np.float64, np.float32], ids=["f64", "f32"])
