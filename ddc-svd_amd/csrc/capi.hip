@@ -797,7 +797,7 @@ static int bidiag_host(int m, int n, double* A, double* alpha, double* beta) {
 }
 
 static int bdsvd_host(int n, const double* alpha, const double* beta, double* sigma,
-                      int refine, double* X, double* Y) {
+                      int refine, double* X, double* Y, int pairs = 0) {
   if (n < 1 || !alpha || !sigma || (n > 1 && !beta)) {
     set_err("invalid arguments");
     return DDC_E_ARG;
@@ -853,7 +853,7 @@ static int bdsvd_host(int n, const double* alpha, const double* beta, double* si
     double* Vt = ws.take<double>((size_t)ldb * n * 2);
     double* Ut = Vt + (size_t)ldb * n;
     double* tmp = ws.take<double>((size_t)n * n);
-    DDC_TRY(twisted_run(n, da, db, ds, Vt, Ut, ldb, ws, st));
+    DDC_TRY(twisted_run(n, da, db, ds, Vt, Ut, ldb, ws, st, pairs));
     if (X) {
       DDC_TRY(transpose_f64(n, n, Vt, ldb, tmp, n, st));
       DDC_TRY(copy_d2h(X, D * n, tmp, D * n, D * n, n, st));
@@ -1166,6 +1166,15 @@ int ddc_test_bidiag(int m, int n, void* A, int f32, double* alpha, double* beta,
                      : test_bidiag(m, n, static_cast<double*>(A), alpha, beta, &form, ms);
   *stopped = form.stopped;
   return rc;
+}
+
+// bdsvd_vectors_gpu with pairs (1 or 2) pairs of waves per group of values.
+int ddc_test_vectors(int n, const double* alpha, const double* beta, double* sigma, double* X,
+                     double* Y, int pairs) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_err[0] = 0;
+  if (!X || !Y || pairs < 1 || pairs > 2) return DDC_E_ARG;
+  return bdsvd_host(n, alpha, beta, sigma, 1, X, Y, pairs);
 }
 
 }  // extern "C"

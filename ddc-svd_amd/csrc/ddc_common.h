@@ -163,10 +163,11 @@ int dc_run(int n, const double* a, const double* b, double* sigma, Arena& ws,
 // Singular vectors of the n x n upper bidiagonal (a[n], b[n-1]) for the
 // ascending singular values sigma (refined in place to high relative
 // accuracy).  Vectors are written sigma-minor: Vt[j*ldv + i] = v_i[j] and
-// Ut[j*ldv + i] = u_i[j], so B v_i = sigma_i u_i.
+// Ut[j*ldv + i] = u_i[j], so B v_i = sigma_i u_i.  pairs (tests): pairs of waves
+// per group of 64 values, 1 or 2; 0 by n.
 void twisted_plan(ArenaPlan& p, int n);
 int twisted_run(int n, const double* a, const double* b, double* sigma,
-                double* Vt, double* Ut, int ldv, Arena& ws, hipStream_t st);
+                double* Vt, double* Ut, int ldv, Arena& ws, hipStream_t st, int pairs = 0);
 
 // U = Q_left [Yb; 0] (m x n) and V = Q_right Xb (n x n) from the reflectors
 // stored in A (m x n, lda), where Yb/Xb are given sigma-minor as from

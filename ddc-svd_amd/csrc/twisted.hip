@@ -1273,7 +1273,7 @@ void twisted_plan(ArenaPlan& p, int n) {
 }
 
 int twisted_run(int n, const double* a, const double* b, double* sigma,
-                double* Vt, double* Ut, int ldv, Arena& ws, hipStream_t st) {
+                double* Vt, double* Ut, int ldv, Arena& ws, hipStream_t st, int pairs) {
   if (n < 1 || ldv < n) return DDC_E_ARG;
   double* qd = ws.take<double>(6 * (size_t)n);
   double* scr = ws.take<double>(2 * tw_ck_size(n));
@@ -1361,7 +1361,8 @@ int twisted_run(int n, const double* a, const double* b, double* sigma,
   // four against two waves: n = 8192, 256 groups, 10.1 and 14.1 ms; n = 12288,
   // 384 groups, 74 and 20.9 ms).
   const unsigned ng = 2 * (unsigned)ceil_div(n, 64);
-  if (ng <= TW_CUS)
+  if (pairs == 0) pairs = ng <= TW_CUS ? 2 : 1;
+  if (pairs == 2)
     hipLaunchKernelGGL(tw_solve<2>, dim3(ng), dim3(256), 0, st, t);
   else
     hipLaunchKernelGGL(tw_solve<1>, dim3(ng), dim3(128), 0, st, t);
