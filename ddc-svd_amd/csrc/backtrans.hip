@@ -232,7 +232,7 @@ __global__ __launch_bounds__(512) void bt_tmerge(int nb, int s, const double* G,
   }
 }
 
-static int form_t(int nb, const double* G, double* T, hipStream_t st) {
+int form_t(int nb, const double* G, double* T, hipStream_t st) {
   static_assert(NBB <= 512, "bt_tmerge joins blocks of up to 256");
   const unsigned nt = (unsigned)ceil_div(nb, TB);
   hipLaunchKernelGGL(bt_tdiag, dim3(nt, nt), dim3(256), 0, st, nb, G, T);

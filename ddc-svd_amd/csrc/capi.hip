@@ -1177,4 +1177,23 @@ int ddc_test_vectors(int n, const double* alpha, const double* beta, double* sig
   return bdsvd_host(n, alpha, beta, sigma, 1, X, Y, pairs);
 }
 
+// T (host, nb x nb) from G (host): form_t.
+int ddc_test_form_t(int nb, const double* G, double* T) {
+  std::lock_guard<std::mutex> lk(g_mu);
+  g_err[0] = 0;
+  if (nb < 1 || nb > 512 || !G || !T) return DDC_E_ARG;
+  DDC_TRY(ctx_init());
+  hipStream_t st = g_ctx.st;
+  ArenaPlan plan;
+  plan.add<double>((size_t)nb * nb * 2);
+  Arena ws;
+  DDC_TRY(arena_get(plan.bytes, ws, st));
+  double* g = ws.take<double>((size_t)nb * nb * 2);
+  if (!g) return DDC_E_NOMEM;
+  const size_t w = sizeof(double) * nb;
+  DDC_TRY(copy_h2d(g, w, G, w, w, nb, st));
+  DDC_TRY(form_t(nb, g, g + (size_t)nb * nb, st));
+  return copy_d2h(T, w, g + (size_t)nb * nb, w, w, nb, st);
+}
+
 }  // extern "C"

@@ -169,6 +169,10 @@ void twisted_plan(ArenaPlan& p, int n);
 int twisted_run(int n, const double* a, const double* b, double* sigma,
                 double* Vt, double* Ut, int ldv, Arena& ws, hipStream_t st, int pairs = 0);
 
+// The triangular factor T (nb x nb, nb <= 512, zeros below the diagonal) of a
+// block of unit-norm reflectors: T^{-1} = I/2 + strict_upper(G).
+int form_t(int nb, const double* G, double* T, hipStream_t st);
+
 // U = Q_left [Yb; 0] (m x n) and V = Q_right Xb (n x n) from the reflectors
 // stored in A (m x n, lda), where Yb/Xb are given sigma-minor as from
 // twisted_run (ld ldb).  U gets leading dimension ldu, V ldv.
