@@ -88,12 +88,12 @@ constexpr int RS_RING = 2;            // steps the boxes hold
 constexpr int RS_XRING = 4;           // steps the areas of x hold
 constexpr int RS_LAUNCH = 15;         // launches of one bidiagonalization at most
 constexpr int RS_SYNC = 16 * RS_LAUNCH + 1;  // sync words
-// The rendezvous' wait, in ticks of the 100 MHz clock: 1 ms.  The work-groups of a
-// free GPU start within some tens of microseconds; where others hold its CUs,
-// those that wait hold CUs themselves, so what is lost to both is kept small
-// beside the panel kernels' time (a bound of 100,000 polls lasted 30 ms in a
-// call of 3.1 ms).
-constexpr int RS_RDV = 100000;
+// The rendezvous' wait in polls: 0.9 ms, with the work-groups of one XCD or of all.
+// Those of a free GPU start within some tens of microseconds; where other work
+// holds its CUs, those that wait hold CUs themselves, so what is lost to both is
+// kept small beside the panel kernels' time (100,000 polls lasted 30 ms in a call
+// of 3.1 ms).  A bound by the clock, read in this loop, cost every launch 4 us.
+constexpr int RS_RDV = 3000;
 constexpr int RS_POLLS = 1 << 21;     // polls of one exchange before it is given up
 // before the first poll of message 1, in units of 64 cycles: it cannot have
 // come sooner (polls in flight delay it: two of them staggered by half a
@@ -281,8 +281,7 @@ __global__ __launch_bounds__(RS_T, 1) void bd_resident(ResArgs<TS> g) {
       unsigned* state = arrived + 1;
       if (go) {
         if (atomicAdd(arrived, 1u) + 1 == g.groups) atomicCAS(state, 0u, RS_GO);
-        const long long t0 = wall_clock64();
-        while (take(state) == 0 && wall_clock64() - t0 < RS_RDV) __builtin_amdgcn_s_sleep(8);
+        for (int i = 0; i < RS_RDV && take(state) == 0; ++i) __builtin_amdgcn_s_sleep(8);
         // all decide alike: whoever writes the state first decides
         atomicCAS(state, 0u, RS_STOP);
         go = take(state) == RS_GO;
