@@ -1102,11 +1102,10 @@ static int bj_time(svd_gpu_batch* p, const BjConfig& c, const void* dA, void* dS
 //      0.70 | 0.65);
 //      all of more than 128 rows: one width and one result, 0 to 5% in favour of
 //      the kernel that holds it alone (8000 of 200 x 8 0.482 | 0.458).
-//  * FP32: the same lines.  2000 of 8 x 8 0.149 | 0.114, of 200 x 8 0.155 | 0.140;
-//    512 of 24 x 24 0.54 | 0.35, 1024 0.58 | 0.67; 1000 up to 40 x 40 (load 0.65)
-//    0.59 | 0.49, 3000 (1.99) 0.80 | 1.24; 256 of 48 x 48 0.48 | 0.53, 512 of
-//    96 x 96 3.05 | 3.10; 10,000 up to 128 13.3 | 15.7, 2000 of 128 x 128
-//    16.6 | 22.2; the other way by at most a seventh (1000 up to 64 0.95 | 0.82).
+//  * FP32: blocks of 8 wherever the matrices of up to 128 rows and more than 8
+//    columns count (10,000 up to 128 13.3 | 15.7, 2000 of 128 x 128 16.6 | 22.2;
+//    1536 of 24 x 24 0.58 | 0.77, but 512 0.54 | 0.35); up to 8 columns of 4 (2000
+//    of 8 x 8 0.149 | 0.114, one 0.082 | 0.056, 2000 of 200 x 8 0.155 | 0.140).
 //    Where one of more than 224 rows outlasts the others the two are within 1%
 //    (150 up to 256 12.1 | 12.0, 600 12.7 | 12.8, 2,500 19.6 | 19.5), so the line
 //    between them costs nothing wherever it lies.
@@ -1120,7 +1119,8 @@ static int bj_variant(const svd_gpu_batch* p) {
     cols = std::max(cols, nt);
     most = std::max(most, (double)nt * nt * mt);
   }
-  if (p->dtype == SVD_GPU_F32 && rows > 224 && p->work < 350.0 * most) return 1;
+  if (p->dtype == SVD_GPU_F32)
+    return cols <= 8 || (rows > 224 && p->work < 350.0 * most) ? 1 : 0;
   const bool few = p->count <= 2 * p->cus || p->work < 0.6 * p->cus * most;
   return cols <= 8 || least > 128 || (cols <= 40 && few) ? 1 : 0;
 }

@@ -68,11 +68,10 @@ def test_tuning_leaves_the_bits(ddcsvd, dtype, count, hi):
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("count,m,n,variant", [
-    (1, 8, 8, 1), (2000, 8, 8, 1), (2000, 9, 9, 0), (300, 8, 128, 1), (512, 24, 24, 1),
-    (2000, 24, 24, 0), (512, 40, 40, 1), (512, 41, 41, 0), (64, 129, 20, 1), (2000, 128, 20, 0)])
-def test_block_width_by_sizes(ddcsvd, dtype, count, m, n, variant):
-    """Matrices of few columns, and small ones that leave CUs idle, take blocks of
-    4 in both types: blocks of 8 leave most of a matrix's waves nothing."""
+    (1, 8, 8, 1), (2000, 8, 8, 1), (300, 8, 128, 1), (500, 200, 8, 1), (2000, 9, 9, 0),
+    (2000, 128, 20, 0)])
+def test_few_columns_take_narrow_blocks(ddcsvd, dtype, count, m, n, variant):
+    """In both types: a block of 8 leaves most of a matrix's waves nothing."""
     from ddcsvd.batched import BatchedSvd
     gpu_case(f"batched width {dtype} {count} of {m} x {n}")
     b = BatchedSvd([m] * count, [n] * count, dtype)
