@@ -69,6 +69,10 @@ constexpr unsigned TW_CUS = 256;    // CUs of the GPU
 constexpr int TW_CK = 64;          // checkpoint interval = LDS chunk
 constexpr int TW_MAXBIS = 200;     // bisection steps per lane at most
 constexpr double TW_CONV = 32.0;   // Rayleigh correction accepted below TW_CONV eps lam
+constexpr double TW_FAR = 0x1p-10;  // corrections above TW_FAR lam are no rounding
+constexpr int TW_IT = 10;           // Rayleigh steps at most
+// the same of a lane whose correction is above TW_FAR lam (a zero's always is)
+constexpr int TW_ITFAR = 30;
 
 enum { TW_UNRES = 1 };
 
@@ -479,7 +483,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
   double nz2 = 1.0, corr = 0.0, prev = INFINITY;
   int rfin = g1 - 1;
   bool active = live;
-  for (int it = 0; it < 10; ++it) {
+  for (int it = 0; it < TW_ITFAR; ++it) {
     if (__ballot(active) == 0) break;  // the same in all waves
     // pass 1: stationary (wave 0, ascending) and progressive (wave 1,
     // descending) transforms with checkpoints
@@ -705,9 +709,14 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
     // includes the correction), the vector's norm saturated, or (from the
     // third step on) the correction no longer halving -- it has reached the
     // rounding floor of gamma_r, which for small singular values sits above
-    // eps*lam
+    // eps*lam.  Not so where the bracket is wide and the steps still large:
+    // beside values of the rounding level (rank-deficient matrices) the first
+    // steps may not halve, and a lane that stopped there kept a vector between
+    // its own and its neighbour's (0.09 to 0.5 from orthogonal).
+    const bool far = !unres && fabs(corr) > TW_FAR * lam && hi - lo > TW_FAR * lam;
     if (lam < 0.0 || fabs(corr) <= TW_CONV * TW_EPS * lam || nz2 > 1.0 / (TW_EPS * TW_EPS) ||
-        (it >= 2 && fabs(corr) > 0.5 * prev)) {
+        (it >= 2 && fabs(corr) > 0.5 * prev && !far) ||
+        it >= (far && lo > 0.0 ? TW_ITFAR : TW_IT) - 1) {
       active = false;
       continue;
     }

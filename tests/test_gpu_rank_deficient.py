@@ -1,0 +1,38 @@
+"""GPU tests of the vectors of rank-deficient matrices: singular values of the
+rounding level, of which several share a block of the bidiagonal with the large
+ones.
+
+The bidiagonals are LAPACK's dgebrd of the matrices.  Values whose relative gap
+in sigma^2 is just above 1e-6 get vectors of their own, accurate to
+eps / 1e-6 = 2e-10; 1e-9 leaves room for a handful of such pairs.
+"""
+import numpy as np
+import pytest
+
+from conftest import gpu_case
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ddcsvd, po, A):
+    _, a, b, _, _ = po.lapack_dgebrd(np.asfortranarray(A))
+    s, X, Y = ddcsvd.bdsvd_vectors(a, b)
+    eye = np.eye(len(a))
+    assert np.linalg.norm(X.T @ X - eye) <= 1e-9
+    assert np.linalg.norm(Y.T @ Y - eye) <= 1e-9
+    B = np.diag(a) + np.diag(b, 1)
+    assert np.linalg.norm(B @ X - Y * s) <= 1e-12 * np.linalg.norm(B)
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 146, 147, 169, 170])
+@pytest.mark.parametrize("kind", ["normal", "binary"])
+def test_products_of_low_rank(ddcsvd, po, kind, seed):
+    rng = np.random.default_rng(seed)
+    n = int(rng.integers(20, 300))
+    m, k = n + int(rng.integers(0, 100)), int(rng.integers(1, n))
+    gpu_case(f"rank deficient {kind} {m} x {n} rank {k} seed {seed}")
+    if kind == "normal":
+        A = rng.standard_normal((m, k)) @ rng.standard_normal((k, n))
+    else:
+        A = (rng.integers(0, 2, (m, k)) @ rng.integers(0, 2, (k, n))).astype(float)
+    _check(ddcsvd, po, A)
