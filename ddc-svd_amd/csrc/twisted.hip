@@ -472,14 +472,27 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
 
   double lam = fmin(fmax(sig * sig, lo), hi);
   // A value whose square is within the pivot guard (0 in particular) is
-  // solved at a shift just below zero (eps^2 smax^2, at least 4 pivmin so
+  // solved at a shift just below zero (at least 4 pivmin so
   // that it is not itself guarded), where the shifted Gram
   // matrix is positive definite: at a shift of exactly 0 a zero diagonal
   // entry makes the transforms' quotients 0/0 (taken as 0 by the guard
   // instead of their limit), every twist index ties and the vector is
-  // wrong.  Its first vector is kept.  (Larger tiny values keep their own
+  // wrong.  The shift is eps^2 smax^2, or eps times the next larger square
+  // where that is less: a zero among values of the rounding level came out
+  // mixed with them (0.2 to 0.8 from orthogonal).  Its first vector is kept,
+  // unless its Rayleigh quotient shows a value far from zero (one that divide
+  // and conquer rounded to zero).  (Larger tiny values keep their own
   // shift: in a graded block they are resolved to high relative accuracy.)
-  if (lam <= pivmin) lam = -fmax(TW_EPS * TW_EPS * smax * smax, 4.0 * pivmin);
+  if (lam <= pivmin) {
+    int j0 = li, j1 = n;  // the brackets' ends rise with the values
+    while (j1 - j0 > 1) {
+      const int j = (j0 + j1) / 2;
+      if (a.lam_lo[j] > pivmin) j1 = j;
+      else j0 = j;
+    }
+    const double next = j1 < n ? a.lam_lo[j1] : smax * smax;
+    lam = -fmax(TW_EPS * fmin(TW_EPS * smax * smax, next), 4.0 * pivmin);
+  }
   double nz2 = 1.0, corr = 0.0, prev = INFINITY;
   int rfin = g1 - 1;
   bool active = live;
@@ -703,7 +716,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
     }
     if (!active) continue;
     corr = gbest / nz2;
-    // converged: a value at the zero floor (lam < 0, its first vector), a
+    // converged: a value of zero (lam < 0, its first vector), a
     // correction within a few ulps of lam (the shift's error is
     // then far below any gap the vector can resolve, and the value returned
     // includes the correction), the vector's norm saturated, or (from the
@@ -714,7 +727,8 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
     // steps may not halve, and a lane that stopped there kept a vector between
     // its own and its neighbour's (0.09 to 0.5 from orthogonal).
     const bool far = !unres && fabs(corr) > TW_FAR * lam && hi - lo > TW_FAR * lam;
-    if (lam < 0.0 || fabs(corr) <= TW_CONV * TW_EPS * lam || nz2 > 1.0 / (TW_EPS * TW_EPS) ||
+    const bool zero = lam < 0.0 && (unres || !(corr > -lam / TW_FAR));
+    if (zero || fabs(corr) <= TW_CONV * TW_EPS * lam || nz2 > 1.0 / (TW_EPS * TW_EPS) ||
         (it >= 2 && fabs(corr) > 0.5 * prev && !far) ||
         it >= (far && lo > 0.0 ? TW_ITFAR : TW_IT) - 1) {
       active = false;
@@ -724,7 +738,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
     // cnt = number of eigenvalues below lam: keep the bracket around idx
     // (an inseparable cluster's bracket is already at the rounding level)
     if (!unres) {
-      if (cnt <= idx) lo = lam; else hi = lam;
+      if (cnt <= idx) lo = fmax(lo, lam); else hi = lam;
     }
     double nl = lam + corr;
     if (!(nl > lo && nl < hi)) nl = 0.5 * (lo + hi);

@@ -36,3 +36,19 @@ def test_products_of_low_rank(ddcsvd, po, kind, seed):
     else:
         A = (rng.integers(0, 2, (m, k)) @ rng.integers(0, 2, (k, n))).astype(float)
     _check(ddcsvd, po, A)
+
+
+@pytest.mark.parametrize("seed", [2, 3, 23, 29, 31, 32, 63, 68, 80, 84, 114])
+def test_zeros_beside_values_of_the_rounding_level(ddcsvd, po, seed):
+    """A third of the rows and columns zero and one column twice: the bidiagonal
+    holds exact zeros next to values down to eps^2 of the largest."""
+    rng = np.random.default_rng(seed)
+    n = int(rng.integers(20, 300))
+    m = n + int(rng.integers(0, 100))
+    gpu_case(f"rank deficient, zero rows and columns {m} x {n} seed {seed}")
+    rng.integers(1, n)
+    A = rng.standard_normal((m, n))
+    A[:, rng.permutation(n)[:n // 3]] = 0
+    A[:, n // 2] = A[:, 0]
+    A[rng.permutation(m)[:m // 3]] = 0
+    _check(ddcsvd, po, A)
