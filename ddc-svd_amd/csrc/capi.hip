@@ -175,9 +175,8 @@ static int arena_get(size_t bytes, Arena& ws, hipStream_t st) {
 // A copy from or to pageable memory goes through two pinned staging buffers:
 // the CPU copies one slice between the caller's buffer and a staging buffer
 // while the DMA engine moves the other.  A pageable hipMemcpy2D with a pitch
-// moves its columns one by one, which was most of a small call: svd_gpu of
-// 640 x 480 takes 3.9 ms (17.7 with direct copies), of 96 x 64 1.15 (2.9),
-// bidiag_gpu of 2048 x 1536 8.9 (33.3), of 640 x 480 2.0 (9.6).
+// moves its columns one by one, which was most of a call: svd_gpu of 640 x 480
+// takes 3.4 ms (17.4 with direct copies), bidiag_gpu of 2048 x 1536 9.6 (34.7).
 
 constexpr size_t STAGE_BYTES = size_t(32) << 20;  // per staging buffer, at most
 constexpr size_t STAGE_SLICE = size_t(1) << 20;   // slices of a copy, at least
@@ -904,7 +903,6 @@ static int backward_dev(int m, int n, const double* U, int ldu, const double* si
   return DDC_OK;
 }
 
-// host buffers: A (m x n, reflectors as bidiag_gpu leaves them) -> Q
 // The bidiagonalization alone by a given form, for the tests: A (m x n, host,
 // FP64 or FP32 storage) is replaced by the reflectors; *ms: its time on the
 // device.
@@ -944,6 +942,7 @@ static int test_bidiag(int m, int n, TS* A, double* alpha, double* beta, BidiagF
   return DDC_OK;
 }
 
+// host buffers: A (m x n, reflectors as bidiag_gpu leaves them) -> Q
 static int form_host(bool left, int m, int n, const double* A, double* Q) {
   DDC_TRY(check_dims(m, n));
   if (m < n) {

@@ -150,12 +150,12 @@ void svd_device_plan(ArenaPlan& p, int m, int n);
 int svd_device(int m, int n, const double* dA, int lda, double* dsigma, double* dU, int ldu,
                double* dV, int ldv, Arena& ws, hipStream_t st);
 
-// Singular values (ascending) of the n x (n+1) upper bidiagonal with diagonal
-// a[n] and super-diagonal b[n] by divide and conquer.
 // bytes (at most 4096) of device memory to the host through a pinned buffer,
 // after the work before them on st; waits for st
 int host_read(void* dst, const void* src, size_t bytes, hipStream_t st);
 
+// Singular values (ascending) of the n x (n+1) upper bidiagonal with diagonal
+// a[n] and super-diagonal b[n] by divide and conquer.
 void dc_plan(ArenaPlan& p, int n);
 int dc_run(int n, const double* a, const double* b, double* sigma, Arena& ws,
            hipStream_t st);

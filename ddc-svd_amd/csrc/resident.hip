@@ -771,15 +771,15 @@ void resident_plan(ArenaPlan& p) {
   p.add<unsigned>(RS_SYNC);
 }
 
-// Column steps k0 .. min(m, n) - 1 of the bidiagonalization of A, whose
-// block A[k0:m, k0:n] must be fully updated.  *done: the steps completed
-// (less than min(m, n) if a launch did not assemble; A is then fully updated
-// from *done, a multiple of align, on).
 __global__ __launch_bounds__(1024) void rs_clear(unsigned* sync, double* beta, int nb) {
   for (int i = threadIdx.x; i < RS_SYNC; i += 1024) sync[i] = 0;
   for (int i = threadIdx.x; i < nb; i += 1024) beta[i] = 0.0;
 }
 
+// Column steps k0 .. min(m, n) - 1 of the bidiagonalization of A, whose
+// block A[k0:m, k0:n] must be fully updated.  *done: the steps completed
+// (less than min(m, n) if a launch did not assemble; A is then fully updated
+// from *done, a multiple of align, on).
 template <typename TS>
 int resident_run(int m, int n, TS* A, int lda, double* alpha, double* beta, int k0, int align,
                  Arena& ws, hipStream_t st, int* done, int absent) {
