@@ -416,8 +416,15 @@ __global__ void k_scale(int m, int n, double* A, int lda, double s1, double s2) 
   }
 }
 
+// Magnitudes (binary exponent of the largest entry) that are not scaled.  The
+// vectors stage multiplies two squares of sigma, of the largest value and of the
+// smallest that counts (eps^2 times that): 2^(4 SCALE_EXP + 104) has to be far from
+// the ends of the range.  (At 450 it left NaN or wrong vectors for entries of
+// 1e80 to 1e135 and 1e-135 to 1e-80.)
+constexpr int SCALE_EXP = 100;
+
 // Checks the m x n device matrix A for NaN and Inf (*nonfinite) and, when
-// its largest entry lies outside [2^-450, 2^450], scales it in place by a
+// its largest entry lies outside [2^-SCALE_EXP, 2^SCALE_EXP], scales it in place by a
 // power of two (exact) into [1/2, 1): *aexp is then the binary exponent
 // that undoes it (x 2^aexp), else 0.  With src (ld lds) A is first filled
 // from it, its rows from m to lda with zeros.  flag: 4 ints of device scratch.
@@ -443,7 +450,7 @@ static int check_and_scale(int m, int n, double* A, int lda, int* flag, hipStrea
   std::memcpy(&amx, &abits, sizeof(amx));
   int e = 0;
   if (amx > 0.0) (void)std::frexp(amx, &e);
-  if (!*nonfinite && amx > 0.0 && (e < -450 || e > 450)) {
+  if (!*nonfinite && amx > 0.0 && (e < -SCALE_EXP || e > SCALE_EXP)) {
     hipLaunchKernelGGL(k_scale, dim3(1024), dim3(256), 0, st, m, n, A, lda,
                        std::ldexp(1.0, -e / 2), std::ldexp(1.0, -e - (-e / 2)));
     DDC_LAUNCHED();
@@ -547,9 +554,9 @@ struct Timer {
 static int tall_stages(int m, int n, TallBufs& b, Arena& ws, double* dU, int ldu,
                        double* dV, int ldv, hipStream_t st, Timer& tm, const double* src = nullptr,
                        int lds = 0) {
-  // A matrix whose largest entry lies outside [2^-450, 2^450] is scaled by
-  // a power of two: the values and vectors stages work with sigma^2, which
-  // would underflow or overflow.  sigma is scaled back at the end; U and V
+  // A matrix whose largest entry lies outside [2^-SCALE_EXP, 2^SCALE_EXP] is scaled by
+  // a power of two: the values and vectors stages work with products of sigma^2,
+  // which would underflow or overflow.  sigma is scaled back at the end; U and V
   // do not change.
   bool nonfinite = false;
   int aexp = 0;
@@ -820,15 +827,15 @@ static int bdsvd_host(int n, const double* alpha, const double* beta, double* si
   double* da = ws.take<double>(n);
   double* db = ws.take<double>(n);
   double* ds = ws.take<double>(n);
-  // a bidiagonal whose largest entry lies outside [2^-450, 2^450] is scaled
-  // by a power of two (exact, in two factors) and sigma scaled back, as in
-  // the SVD: the values and vectors stages work with sigma^2
+  // a bidiagonal whose largest entry lies outside [2^-SCALE_EXP, 2^SCALE_EXP] is
+  // scaled by a power of two (exact, in two factors) and sigma scaled back, as in
+  // the SVD
   double amx = 0.0;
   for (int i = 0; i < n; ++i) amx = std::fmax(amx, std::fabs(alpha[i]));
   for (int i = 0; i + 1 < n; ++i) amx = std::fmax(amx, std::fabs(beta[i]));
   int aexp = 0;  // stays 0 for a zero or non-finite bidiagonal
   if (amx > 0.0 && std::isfinite(amx)) (void)std::frexp(amx, &aexp);
-  const bool scaled = aexp < -450 || aexp > 450;
+  const bool scaled = aexp < -SCALE_EXP || aexp > SCALE_EXP;
   std::vector<double> sa, sb;
   const double* pa = alpha;
   const double* pb = beta;
