@@ -89,10 +89,14 @@ __device__ __forceinline__ double keep(double x) {
   asm("" : "+v"(x));
   return x;
 }
-// stationary qd step: s_{i+1} from s_i (lld_i = 0 is a block boundary)
-__device__ __forceinline__ double stat_next(double s, double dp, double lld, double lam) {
+// stationary qd step: s_{i+1} from s_i (lld_i = 0 is a block boundary; at
+// d_i = 0 the quotient s_i / D+_i is 1, which 0/0 and the guard would make 0: the
+// counts and vectors of bidiagonals with zeros on the diagonal went wrong where
+// a shift met an eigenvalue of a leading block, as integer matrices have them)
+__device__ __forceinline__ double stat_next(double s, double dp, double d, double lld,
+                                            double lam) {
   const double q = keep(lld * s / dp);
-  return lld == 0.0 ? -lam : q - lam;
+  return (lld == 0.0 || d == 0.0 ? lld : q) - lam;
 }
 // progressive qd step: p_i from p_{i+1}
 __device__ __forceinline__ double prog_prev(double p, double d, double dm, double lld, double lam) {
@@ -242,8 +246,8 @@ __device__ __forceinline__ void sturm2(const double* d, const double* lld, int n
     const double p0 = guard(di + s0, pivmin), p1 = guard(di + s1, pivmin);
     k0 += p0 < 0.0;
     k1 += p1 < 0.0;
-    s0 = stat_next(s0, p0, li, x0);
-    s1 = stat_next(s1, p1, li, x1);
+    s0 = stat_next(s0, p0, di, li, x0);
+    s1 = stat_next(s1, p1, di, li, x1);
   }
   c0 = x0 > 0.0 ? k0 : 0;
   c1 = x1 > 0.0 ? k1 : 0;
@@ -257,7 +261,7 @@ __device__ __forceinline__ int sturm1(const double* d, const double* lld, int n,
   for (int i = 0; i < n; ++i) {
     const double p = guard(d[i] + s, pivmin);
     k += p < 0.0;
-    s = stat_next(s, p, lld[i], x);
+    s = stat_next(s, p, d[i], lld[i], x);
   }
   return x > 0.0 ? k : 0;
 }
@@ -337,8 +341,8 @@ __global__ __launch_bounds__(256) void tw_isolate(IsoArgs A) {
       const double p0 = guard(di + s0, pivmin), p1 = guard(di + s1, pivmin);
       k0 += p0 < 0.0;
       k1 += p1 < 0.0;
-      s0 = stat_next(s0, p0, li, lo);
-      s1 = stat_next(s1, p1, li, hi);
+      s0 = stat_next(s0, p0, di, li, lo);
+      s1 = stat_next(s1, p1, di, li, hi);
       const int e = A.be[i];
       if (e == i + 1) {
         const int mb = (hi > 0.0 ? k1 : 0) - (lo > 0.0 ? k0 : 0);
@@ -513,7 +517,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
           auto step = [&](int e) {
             const double dp = guard(qd_d[e] + s, pivmin);
             cnt += (dp < 0.0);
-            s = stat_next(s, dp, qd_lld[e], lam);  // past the last index: unused
+            s = stat_next(s, dp, qd_d[e], qd_lld[e], lam);  // past the last index: unused
           };
           if (len == TW_CK) {
 #pragma unroll 8
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
         auto step = [&](int e) {
           bw[e][lane] = ss;
           const double dp = guard(qd_d[e] + ss, pivmin);
-          ss = stat_next(ss, dp, qd_lld[e], lam);
+          ss = stat_next(ss, dp, qd_d[e], qd_lld[e], lam);
         };
         if (len == TW_CK) {
 #pragma unroll 8
@@ -655,7 +659,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
           auto step = [&](int e) {
             const double dp = guard(qd_d[e] + ss, pivmin);
             bw[e][lane] = -(qd_ld[e] / dp);
-            ss = stat_next(ss, dp, qd_lld[e], lam);
+            ss = stat_next(ss, dp, qd_d[e], qd_lld[e], lam);
           };
           if (ns == TW_CK) {
 #pragma unroll 8
@@ -915,7 +919,7 @@ __global__ __launch_bounds__(256) void tw_rr(RrArgs A) {
             vec[vi(i)] = w / dp;
             lprev = qs[rep][1][e] / dp;
             wprev = w;
-            s = stat_next(s, dp, qs[rep][2][e], tau);
+            s = stat_next(s, dp, qs[rep][0][e], qs[rep][2][e], tau);
           }
         }
       }
@@ -936,7 +940,7 @@ __global__ __launch_bounds__(256) void tw_rr(RrArgs A) {
           for (int e = 0; e < len; ++e) {
             const double dp = guard(qs[rep][0][e] + ss, pm);
             buf[rep][e][lane] = qs[rep][1][e] / dp;  // L+_i
-            ss = stat_next(ss, dp, qs[rep][2][e], tau);
+            ss = stat_next(ss, dp, qs[rep][0][e], qs[rep][2][e], tau);
           }
           for (int e = len - 1; e >= 0; --e) {
             const int i = e0 + e;
