@@ -76,6 +76,13 @@ constexpr int TW_ITFAR = 30;
 
 enum { TW_UNRES = 1 };
 
+// The least pivot: a step forms lld s / D+ with s itself up to smax^2 and, one step
+// after a pivot of this size, lld (lld s / pivmin), which must not overflow (two
+// infinities leave a NaN, and the counts behind it are wrong).
+__device__ __forceinline__ double pivot_min(double smax) {
+  const double s2 = fmax(1.0, smax * smax);
+  return 1024.0 * TW_TINY * s2 * s2 * s2;
+}
 __device__ __forceinline__ double guard(double x, double pivmin) {
   return (fabs(x) < pivmin) ? -pivmin : x;
 }
@@ -277,7 +284,7 @@ __global__ __launch_bounds__(256) void tw_isolate(IsoArgs A) {
   const double* d = A.qd;
   const double* lld = A.qd + 2 * (size_t)n;
   const double smax = A.smax, dl = A.dl;
-  const double pivmin = TW_TINY * fmax(1.0, smax * smax);
+  const double pivmin = pivot_min(smax);
   const double top = (smax + dl) * (smax + dl) * (1.0 + 1e-8);
   const int c_s = A.cs[jj], c_e = A.ce[jj];
   double lo = fmax(0.0, A.sig[c_s] - dl);
@@ -465,7 +472,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
   double (*bw)[64] = buf[wave];
 
   const double smax = a.smax;
-  const double pivmin = TW_TINY * fmax(1.0, smax * smax);
+  const double pivmin = pivot_min(smax);
   const double sig = live ? a.sig_in[idx] : 0.0;
   double lo = a.lam_lo[li], hi = a.lam_hi[li];
   const bool unres = (a.flags[li] & TW_UNRES) != 0;
@@ -838,7 +845,7 @@ __global__ __launch_bounds__(256) void tw_rr(RrArgs A) {
   const int64_t ldv = A.ldv;
   const int* mem = A.members + moff;
   const double smax = A.smax;
-  const double pivmin = TW_TINY * fmax(1.0, smax * smax);
+  const double pivmin = pivot_min(smax);
   // a group wider than one window takes its left basis from the right one
   // (phase B), unless its values are at the rounding level of zero
   const bool fromv = gw.z > TW_KMAX && A.sigma[mem[0]] > 1024.0 * TW_EPS * smax;

@@ -32,3 +32,11 @@ def _check(ddcsvd, a, b):
 def test_zeros_on_the_diagonal(ddcsvd, a, b):
     gpu_case(f"bdsvd_vectors {a} {b}")
     _check(ddcsvd, a, b)
+
+
+@pytest.mark.parametrize("seed", range(24))
+def test_random_whole_entries(ddcsvd, seed):
+    rng = np.random.default_rng(seed)
+    n = int(rng.integers(2, 600))
+    gpu_case(f"bdsvd_vectors whole entries n {n} seed {seed}")
+    _check(ddcsvd, rng.integers(-2, 3, n), rng.integers(-2, 3, n - 1))
