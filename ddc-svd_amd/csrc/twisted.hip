@@ -69,7 +69,7 @@ constexpr unsigned TW_CUS = 256;    // CUs of the GPU
 constexpr int TW_CK = 64;          // checkpoint interval = LDS chunk
 constexpr int TW_MAXBIS = 200;     // bisection steps per lane at most
 constexpr double TW_CONV = 32.0;   // Rayleigh correction accepted below TW_CONV eps lam
-constexpr double TW_FAR = 0x1p-10;  // corrections above TW_FAR lam are no rounding
+constexpr double TW_FAR = 0x1p-20;  // corrections above TW_FAR lam are no rounding
 constexpr int TW_IT = 10;           // Rayleigh steps at most
 // the same of a lane whose correction is above TW_FAR lam (a zero's always is)
 constexpr int TW_ITFAR = 30;
