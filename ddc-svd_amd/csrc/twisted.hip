@@ -69,7 +69,7 @@ constexpr unsigned TW_CUS = 256;    // CUs of the GPU
 constexpr int TW_CK = 64;          // checkpoint interval = LDS chunk
 constexpr int TW_MAXBIS = 200;     // bisection steps per lane at most
 constexpr double TW_CONV = 32.0;   // Rayleigh correction accepted below TW_CONV eps lam
-constexpr double TW_FAR = 0x1p-20;  // corrections above TW_FAR lam are no rounding
+constexpr double TW_FAR = 0x1p-30;  // corrections above TW_FAR lam are no rounding
 constexpr int TW_IT = 10;           // Rayleigh steps at most
 // the same of a lane whose correction is above TW_FAR lam (a zero's always is)
 constexpr int TW_ITFAR = 30;
@@ -738,7 +738,7 @@ __global__ __launch_bounds__(128 * H) void tw_solve(TwArgs a) {
     // steps may not halve, and a lane that stopped there kept a vector between
     // its own and its neighbour's (0.09 to 0.5 from orthogonal).
     const bool far = !unres && fabs(corr) > TW_FAR * lam && hi - lo > TW_FAR * lam;
-    const bool zero = lam < 0.0 && (unres || !(corr > -lam / TW_FAR));
+    const bool zero = lam < 0.0 && (unres || !(corr > -1024.0 * lam));
     if (zero || fabs(corr) <= TW_CONV * TW_EPS * lam || nz2 > 1.0 / (TW_EPS * TW_EPS) ||
         (it >= 2 && fabs(corr) > 0.5 * prev && !far) ||
         it >= (far && lo > 0.0 ? TW_ITFAR : TW_IT) - 1) {

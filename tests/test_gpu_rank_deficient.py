@@ -52,3 +52,21 @@ def test_zeros_beside_values_of_the_rounding_level(ddcsvd, po, seed):
     A[:, n // 2] = A[:, 0]
     A[rng.permutation(m)[:m // 3]] = 0
     _check(ddcsvd, po, A)
+
+
+@pytest.mark.parametrize("seed,m,n", [(40, 1455, 1451), (81, 773, 766), (129, 725, 688),
+                                      (168, 560, 538), (236, 1981, 1792)])
+@pytest.mark.parametrize("decades", [8, 12, 16])
+def test_graded_columns(ddcsvd, seed, m, n, decades):
+    """Columns falling to 10^-decades of the first: values on both sides of the
+    rounding level in one block, many of them close.  The bound is that of above."""
+    torch = pytest.importorskip("torch")
+    gpu_case(f"graded columns {m} x {n} by 1e-{decades}")
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    A = torch.randn(m, n, dtype=torch.float64, device="cuda", generator=g)
+    A = A * torch.logspace(0, -decades, n, dtype=torch.float64, device="cuda")
+    s, U, V = ddcsvd.svd_torch(A)
+    eye = torch.eye(n, dtype=torch.float64, device="cuda")
+    assert torch.linalg.norm(U.T @ U - eye) <= 1e-9
+    assert torch.linalg.norm(V.T @ V - eye) <= 1e-9
+    assert torch.linalg.norm((U * s) @ V.T - A) <= 1e-12 * torch.linalg.norm(A)
